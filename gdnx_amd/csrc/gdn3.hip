@@ -2039,36 +2039,50 @@ __global__ void __launch_bounds__(kNT) gdn3_compact_kernel(G3CompactArgs p) {
     return;
   }
   // decode batch: only the rows whose token closes a compaction interval.
-  // The chains are strided over a grid of at most kDecCompactGrid
-  // workgroups; a workgroup's threads check up to kNT of its chains at once
-  // and list those that compact (the order of the list does not matter:
-  // the chains are independent), so a step that closes no interval costs
+  // Every workgroup reads all the rows' positions and lists the ones that
+  // compact, in row order; the chains of the listed rows go round the grid
+  // one by one.  A compaction is ~27 us of latency on a workgroup that holds
+  // a CU's LDS, so the launch is as long as the most any workgroup gets:
+  // 1024 due chains of 16384 take 4 each on 256 workgroups, 125 us at d =
+  // 128 (each workgroup checking its own stride of the chains left all 8 of
+  // a stride to one workgroup whenever the rows' positions repeat with a
+  // period that divides it: 220 us).  A step that closes no interval costs
   // one round of position reads.
-  __shared__ int todo[kNT];
-  __shared__ int ntodo;
-  const int K = (p.N - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;   // this workgroup's chains
-  for (int base = 0; base < K; base += kNT) {
-    if (tid == 0) ntodo = 0;
-    __syncthreads();
-    if (base + tid < K) {
-      const int bi = blockIdx.x + (base + tid) * gridDim.x;
-      const int row = bi / p.hm;
+  __shared__ int rows[kNT];
+  __shared__ int wcnt[kNT / 64];
+  const int NS = p.N / p.hm, lane = tid & 63, wave = tid >> 6;
+  long long seen = 0;   // due chains of the rows before this batch
+  for (int base = 0; base < NS; base += kNT) {
+    const int row = base + tid;
+    bool go = false;
+    if (row < NS) {
       const int pos = p.pos[row];
-      bool go = pos >= 0 && (pos + 1) % p.Kc == 0;   // (a negative position is an empty row)
+      go = pos >= 0 && (pos + 1) % p.Kc == 0;   // (a negative position is an empty row)
       if (go && p.slots) {
         const int sl = p.slots[row];
         go = sl >= 0 && sl < p.nslots;
       }
-      if (go) todo[atomicAdd(&ntodo, 1)] = bi;
     }
+    const unsigned long long due = __ballot(go);
+    if (lane == 0) wcnt[wave] = __popcll(due);
     __syncthreads();
-    const int n = ntodo;
-    for (int i = 0; i < n; ++i) {
-      const int bi = todo[i];
-      const int chain = p.slots ? p.slots[bi / p.hm] * p.hm + bi % p.hm : bi;
-      compact_chain<D, P, CT>(p, sm, chain, bi, tid);
+    int at = __popcll(due & ((1ull << lane) - 1)), n = 0;
+#pragma unroll
+    for (int w = 0; w < kNT / 64; ++w) {
+      if (w < wave) at += wcnt[w];
+      n += wcnt[w];
+    }
+    if (go) rows[at] = row;
+    __syncthreads();
+    const long long cnt = (long long)n * p.hm;
+    const int G = gridDim.x;
+    for (long long e = (blockIdx.x + G - seen % G) % G; e < cnt; e += G) {   // due chain seen + e is this workgroup's
+      const int r = rows[e / p.hm], ch = (int)(e % p.hm);
+      compact_chain<D, P, CT>(p, sm, (p.slots ? p.slots[r] : r) * p.hm + ch, r * p.hm + ch, tid);
       __syncthreads();   // the chain's last LDS reads before the next one's loads
     }
+    seen += cnt;
+    __syncthreads();   // rows and wcnt are read before the next batch writes them
   }
 }
 
@@ -2154,12 +2168,24 @@ __global__ void __launch_bounds__(kNT) kron_read_kernel(KronReadArgs p) {
   }
 }
 
-// Workgroups of a decode batch's compaction launch (grid-stride over chains).
-constexpr int kDecCompactGrid = 2048;
+int cu_count() {
+  static int n = 0;
+  if (n == 0) {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) ==
+                                                hipSuccess && v > 0)
+      n = v;
+    else
+      n = 256;
+  }
+  return n;
+}
 
 template <int D, int P>
 int launch_compact(const G3CompactArgs& a, hipStream_t stream) {
-  const int grid = a.pos ? (a.N < kDecCompactGrid ? a.N : kDecCompactGrid) : a.N;
+  // a decode batch's due chains go round the workgroups that LDS lets run at once
+  const long long fit = (long long)cu_count() * (160 * 1024 / (int)sizeof(G3CompactSmem<D, P>));
+  const int grid = a.pos ? (int)(a.N < fit ? a.N : fit) : a.N;
   if (a.skron && a.skron_dtype == GDNX_DTYPE_BF16)
     hipLaunchKernelGGL((gdn3_compact_kernel<D, P, bf16>), dim3(grid), dim3(kNT), 0, stream, a);
   else
@@ -2185,19 +2211,6 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // The pipelined window kernel for intervals of several sub-chunks: the
 // value split whose workgroups all run at once (at most two per CU, as LDS
 // allows) with the fewest rounds, the widest among equals
-int cu_count() {
-  static int n = 0;
-  if (n == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) ==
-                                                hipSuccess && v > 0)
-      n = v;
-    else
-      n = 256;
-  }
-  return n;
-}
-
 template <typename CT, int D, int P, int NVB>
 void pipe_score(int N, int& best_nvb, long long& best_rounds) {
   constexpr size_t lds = pipe_lds<CT, D, P, NVB>();

@@ -98,4 +98,31 @@ __host__ __device__ __forceinline__ size_t g3_stash_bytes(int N, int nch, int nc
          g3_align256((size_t)ncomp * N * rmn * 4 + 4);
 }
 
+// The window runs in sub-chunks of kSC = 16 tokens aligned with the slots:
+// the P slots are NB = P / 16 blocks, block b holding slots 16 b .. 16 b + 15.
+// Sub-chunk c (global tokens 16 c .. 16 c + 15) writes block c mod NB.  Token
+// i of it sees the other NB - 1 blocks whole (the writes of sub-chunks c - 1
+// .. c - NB + 1) and, of block c mod NB, the slots p >= i the writes of
+// sub-chunk c - NB still hold; at P = 16 that is the banded previous chunk.
+constexpr int kSC = 16;
+
+// Per-chain offsets of the token-major inputs and outputs
+struct G3Tok {
+  size_t qkv_tok, qkv_base, gate_tok, gate_base, dec_tok, dec_base, y_tok, y_base;
+  int gc;
+  __device__ __forceinline__ G3Tok(const G3FwdArgs& p, int chain, int D) {
+    const int H = p.H, M = p.M, T = p.T, L = p.qkv_lanes;
+    const int b = chain / (H * M), hm = chain % (H * M), h = hm / M, m = hm % M;
+    gc = p.gate_ch;
+    qkv_tok = (size_t)H * L * D;
+    qkv_base = ((size_t)b * T * H + h) * L * D + (L > 1 ? (size_t)m * D : 0);
+    gate_tok = (size_t)H * M * gc;
+    gate_base = (((size_t)b * T * H + h) * M + m) * gc;
+    dec_tok = (size_t)H * M;
+    dec_base = ((size_t)b * T * H + h) * M + m;
+    y_tok = (size_t)H * M * D;
+    y_base = (((size_t)b * T * H + h) * M + m) * D;
+  }
+};
+
 }  // namespace gdnx

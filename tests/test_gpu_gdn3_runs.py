@@ -1,0 +1,59 @@
+"""GDN3 forward over intervals of many sub-chunks, cut into runs: the window
+carried from run to run, the state's keys and writes seen across ragged call
+edges, against the CPU oracle (rel-L2 1e-4 in float32, 1e-2 in bf16, the
+net writes twice that, the keys 1e-5)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from gdnx_amd import gdn3
+from oracle import gdn3 as og
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rel_l2(a, b):
+    a, b = a.double().cpu(), b.double().cpu()
+    return ((a - b).norm() / b.norm().clamp_min(1e-30)).item()
+
+
+# (D, P, K_c, t0, T): the smallest interval the runs take (3 sub-chunks), one
+# batch, a run more than a batch, ragged starts inside a slot block and ends
+# that leave the old writes in a block, intervals of one, two and many runs
+CASES = [(128, 16, 48, 0, 96), (128, 16, 64, 5, 190), (128, 16, 1 << 20, 0, 1100), (64, 16, 512, 23, 1061),
+         (128, 32, 512, 17, 700), (64, 32, 128, 0, 333), (128, 64, 1 << 20, 61, 900), (64, 64, 256, 70, 770),
+         (128, 16, 256, 255, 258), (64, 64, 64 * 5, 3, 45)]
+
+
+@pytest.mark.parametrize("io", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("D,P,Kc,t0,T", CASES)
+def test_runs_match_oracle(gpu_lib, D, P, Kc, t0, T, io):
+    print(f"case: gdn3 runs D={D} P={P} Kc={Kc} t0={t0} T={T} {io}", flush=True)
+    B, H, M, R = 1, 1, 2, 4
+    N = B * H * M
+    f = (16, 16, 8, 8) if D == 128 else (8, 8, 8, 8)
+    g = torch.Generator().manual_seed(D + P + T)
+    q, k = (F.normalize(torch.randn(B, T, H, D, generator=g), dim=-1).to(io) for _ in range(2))
+    v = torch.randn(B, T, H, D, generator=g).to(io)
+    gate = (B, T, H, M, D) if (P + T) % 2 else (B, T, H, M)
+    b, w = (torch.sigmoid(torch.randn(*gate, generator=g)) for _ in range(2))
+    dec = torch.exp(-torch.rand(B, T, H, M, generator=g) * torch.tensor([0.1, 0.002])).clamp(max=1.0)
+    st0 = None
+    if t0:
+        st0 = (torch.randn(N, R, f[0], f[1], generator=g) * 0.2, torch.randn(N, R, f[2], f[3], generator=g) * 0.1,
+               torch.randn(N, D, P, generator=g) * 0.4,
+               F.normalize(torch.randn(N, P, D, generator=g), dim=-1).transpose(1, 2).contiguous())
+    wide = (B, T, H, M, D)
+    ex = [x.double().unsqueeze(3).expand(wide) for x in (q, k, v)]
+    gx = [x.double() if x.dim() == 5 else x.double().unsqueeze(-1).expand(wide) for x in (b, w)]
+    yr, sr, _ = og.gdn3_recurrence(*ex, *gx, dec.double(), R=R, P=P, factors=f, compact_every=Kc,
+                                   sign_mode="canonical", return_state=True, state0=st0, t0=t0)
+    y, s, _ = gdn3.gdn3_recurrent_state(*(x.to(DEV) for x in (q, k, v, b, w, dec)), R=R, P=P, factors=f,
+                                        compact_every=Kc, return_state=True, t0=t0,
+                                        state0=None if st0 is None else tuple(x.to(DEV) for x in st0))
+    torch.cuda.synchronize()
+    tol = 1e-4 if io == torch.float32 else 1e-2
+    assert rel_l2(y, yr) <= tol
+    assert rel_l2(s[2], sr[2]) <= 2 * tol
+    assert rel_l2(s[3], sr[3]) <= 1e-5     # keys decay in float32 from the inputs

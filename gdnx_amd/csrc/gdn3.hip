@@ -24,8 +24,10 @@
 // Kr(x) = (sum_r A_r (x) B_r) x is read on MFMA against the materialised
 // d x d Kronecker matrix, rebuilt after every compaction.
 //
-// One workgroup per chain carries the whole state in LDS; the chunk loop
-// is sequential because every compaction depends on the window it closes.
+// With a compaction after every window one workgroup per chain carries the
+// whole state in LDS (gdn3_fused_kernel); its chunk loop is sequential because
+// every compaction depends on the window it closes.  Longer intervals run in
+// gdn3_long.hip, with a compaction launch between them.
 #include <mutex>
 
 #include "gdn3_common.hpp"
@@ -730,24 +732,6 @@ __device__ __forceinline__ void g3_compact(G3Compact<D, P, STG>& cs, float* ab, 
 // fused forward
 // ---------------------------------------------------------------------------
 
-template <typename CT, int D, int P, int NVB>
-struct G3WinSmem {
-  static constexpr int NB = P / kSC;
-  static constexpr bool KF = sizeof(CT) == 4;  // fp32 IO: the grams read the fp32 window keys
-  alignas(16) CT x[3 * kSC][D + 8];      // rows: H (0..15), Q (16..31), K (32..47)
-  alignas(16) float u[kSC][D + 4];       // w (.) v
-  alignas(16) float kr[2 * kSC][D + 4];  // Kronecker reads of H and Q
-  alignas(16) float pp[4][kSC][kSC + 4]; // H K^T (then inverse scratch), Aq, T, inverse scratch
-  alignas(16) float po[2][kSC][P + 4];   // Ho, Qo over the P slots
-  alignas(16) CT skron[D / NVB][D + 8];  // sum_r A_r (x) B_r, this workgroup's rows v
-  alignas(16) float vbd[P][D + 4];       // window keys: block b decayed to e^{-boff_b} of now
-  alignas(16) CT vbx[KF ? 1 : P][D + 8]; // the same in the compute dtype (bf16 IO)
-  float G[kSC], alpha[kSC], lg[kSC], kco[kSC], qco[kSC], gam[kSC], vsc[kSC];
-  float boff[NB];                        // log decay of block b's keys since they were last rebased
-};
-template <typename CT, int D, int P, int NVB>
-constexpr bool win_fits() { return sizeof(G3WinSmem<CT, D, P, NVB>) <= 160 * 1024; }
-
 template <typename CT> struct W16Of { static constexpr int value = 8 * sizeof(CT) / 16; };
 
 __device__ __forceinline__ void unpack8(const uint4* w, float* f, const bf16*) {
@@ -1251,132 +1235,6 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
     gacc += w.G[kSC - 1];
 }
 
-// Sub-chunks [c0, c1) of one compaction interval (or the tail) for every
-// chain; the window state enters and leaves through the workspace.  A
-// chain's value columns are split over NVB workgroups (D / 16 / NVB value
-// tiles each): the grams, the triangular inverse and the window keys depend
-// on no value column and are formed by each of them; the Kronecker reads, the
-// window algebra, the net writes U and y are split.
-template <typename CT, int D, int P, int NVB>
-__global__ void __launch_bounds__(kNT) gdn3_window_kernel(G3FwdArgs p) {
-  typedef G3WinSmem<CT, D, P, NVB> Sm;
-  __shared__ Sm sm;
-  constexpr int NB = Sm::NB;
-  constexpr int DG = D / 8;  // 8-element load units per token row
-  constexpr int UNITS = kSC * DG;
-  constexpr int W16 = W16Of<CT>::value;
-  constexpr int KS = FragT<CT>::KSTEP;
-  typedef typename FragT<CT>::type Frag;
-  static_assert(UNITS <= kNT && UNITS % 64 == 0, "one load unit per thread");
-  static_assert(P % kSC == 0 && NB >= 1 && NB <= 4, "whole 16-slot blocks, at most 4");
-  static_assert(sizeof(Sm) <= 160 * 1024, "LDS budget");
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g4 = lane >> 4, n16 = lane & 15;
-  const int H = p.H, M = p.M, T = p.T;
-  const int N = p.B * H * M;
-  const int work = xcd_remap(blockIdx.x, N * NVB);   // a chain's NVB workgroups land on one XCD
-  const int chain = work / NVB, vb = work % NVB;
-  typedef G3D<D> Ge;
-  constexpr int NVTW = D / 16 / NVB;   // value tiles of this workgroup: vb NVTW + [0, NVTW)
-  static_assert(NVTW >= 1 && (D / 16) % NVB == 0, "value split");
-
-  const bool has_unit = tid < UNITS;
-  const int ui = tid / DG, ud = 8 * (tid % DG);
-  typedef G3Raw<CT> Raw;
-  const G3Tok tk(p, chain, D);
-  // sub-chunk c covers global tokens [16 c, 16 c + 16): local token 16 c + i - t0
-  auto fetch = [&](Raw& r, int c) { g3_fetch<CT>(p, tk, r, c * kSC + ui - p.t0, has_unit, ud); };
-
-  // window state: zero for the first interval, else from the workspace.
-  // Wave w holds value tiles vtile(a) = vb NVTW + w + 4 a of the workgroup's
-  // (a < VPW, where w + 4 a < NVTW), of every block
-  constexpr int VPW = (NVTW + 3) / 4;
-  auto vown = [&](int a) { return wave + 4 * a < NVTW; };
-  auto vtile = [&](int a) { return vb * NVTW + wave + 4 * a; };
-  f32x4 uo[NB][VPW];
-  float* uw = p.uw + (size_t)chain * P * D;
-  float* vw = p.vw + (size_t)chain * P * D;
-  if (p.first) {
-    for (int e = tid; e < P * (D + 4); e += kNT) (&sm.vbd[0][0])[e] = 0.f;
-    if constexpr (!Sm::KF)
-      for (int e = tid; e < P * (D + 8); e += kNT) (&sm.vbx[0][0])[e] = (CT)0.f;
-#pragma unroll
-    for (int bl = 0; bl < NB; ++bl)
-#pragma unroll
-      for (int a = 0; a < VPW; ++a) uo[bl][a] = zero4();
-  } else {
-    for (int e = tid; e < P * D; e += kNT) {
-      const int j = e / D, d = e % D;
-      const float kv = vw[e];
-      sm.vbd[j][d] = kv;
-      if constexpr (!Sm::KF) sm.vbx[j][d] = from_f<CT>(kv);
-    }
-#pragma unroll
-    for (int bl = 0; bl < NB; ++bl)
-#pragma unroll
-      for (int a = 0; a < VPW; ++a)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          uo[bl][a][s] = vown(a) ? uw[(bl * kSC + 4 * g4 + s) * D + vtile(a) * 16 + n16] : 0.f;
-  }
-  if (tid < NB) sm.boff[tid] = 0.f;
-  const bool live = p.live;
-  if (live) {   // this workgroup's value rows of the Kronecker matrix
-    constexpr int PER = 16 / sizeof(CT);  // elements per 16-byte load
-    const uint4* src = (const uint4*)((const CT*)p.skron + ((size_t)chain * D + vb * NVTW * 16) * D);
-    for (int e = tid; e < NVTW * 16 * D / PER; e += kNT) {
-      const int v = (e * PER) / D, k = (e * PER) % D;   // (local row)
-      *(uint4*)&sm.skron[v][k] = src[e];
-    }
-  }
-  float gacc = 0.f;
-
-  Raw raw;
-  fetch(raw, p.c0);
-  const G3WinView<CT, D, P> w{sm.x, sm.u, sm.kr, sm.pp, sm.po, sm.skron, sm.vbd, sm.vbx, sm.G,
-                              sm.alpha, sm.lg, sm.kco, sm.qco, sm.gam, sm.vsc, sm.boff};
-  for (int c = p.c0; c < p.c1; ++c)
-    g3_window_step<CT, D, P, NVB>(w, p, tk, chain, vb, c, c == p.c0, c + 1 < p.c1 ? c + 1 : -1, live, gacc, uo,
-                                  raw);
-  __syncthreads();
-  if (p.c1 > p.c0 && tid < NB)   // the last sub-chunk's block rebased, the others decayed
-    sm.boff[tid] = (tid == (p.c1 - 1) % NB) ? 0.f : sm.boff[tid] + sm.G[kSC - 1];
-  __syncthreads();
-  // window state out (and the final state after the last sub-chunk): the
-  // value columns from their workgroup, the keys and decays from the first
-#pragma unroll
-  for (int a = 0; a < VPW; ++a) {
-    if (!vown(a)) continue;
-#pragma unroll
-    for (int bl = 0; bl < NB; ++bl)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int i = bl * kSC + 4 * g4 + s, v = vtile(a) * 16 + n16;
-        uw[i * D + v] = uo[bl][a][s];
-        if (p.last && p.U_out) p.U_out[((size_t)chain * D + v) * P + i] = uo[bl][a][s];
-      }
-  }
-  if (vb != 0) return;
-  for (int e = tid; e < P * D; e += kNT) {
-    const int j = e / D, d = e % D;
-    const float kv = sm.vbd[j][d] * expf(sm.boff[j / kSC]);
-    vw[e] = kv;
-    if (p.last && p.Vb_out) p.Vb_out[((size_t)chain * D + d) * P + j] = kv;
-  }
-  if (tid == 0) p.gsum[chain] = gacc;
-  if (p.last && !p.complete) {  // no compaction follows: A, B decayed since the last one
-    // the workspace holds every chain's A [N][R m], then every chain's B [N][R n]
-    const float dk = expf(gacc);
-    const float* af = p.ab + (size_t)chain * Ge::R * Ge::m;
-    const float* bf = p.ab + (size_t)N * Ge::R * Ge::m + (size_t)chain * Ge::R * Ge::n;
-    if (p.A_out)
-      for (int e = tid; e < Ge::R * Ge::m; e += kNT) p.A_out[(size_t)chain * Ge::R * Ge::m + e] = af[e] * dk;
-    if (p.B_out)
-      for (int e = tid; e < Ge::R * Ge::n; e += kNT) p.B_out[(size_t)chain * Ge::R * Ge::n + e] = bf[e] * dk;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // compaction, one chain per block: the chunked forward's step between
 // intervals and the gdnx_gdn3_compact entry point
@@ -1777,33 +1635,6 @@ int compact_dispatch(const G3CompactArgs& a, hipStream_t stream) {
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// value split: ~512 workgroups, two per CU (NVB workgroups per chain, at
-// least one value tile each), or the smallest larger split whose LDS fits
-template <typename CT, int D, int P>
-int launch_window(const G3FwdArgs& a, int N, hipStream_t stream) {
-  constexpr int V2 = D / 16 < 2 ? D / 16 : 2, V4 = D / 16 < 4 ? D / 16 : 4, V8 = D / 16 < 8 ? D / 16 : 8;
-  static_assert(win_fits<CT, D, P, V8>(), "the widest split fits");
-  const int nvb = N >= 512 ? 1 : N >= 256 ? V2 : N >= 128 ? V4 : V8;
-  bool done = false;
-  if constexpr (win_fits<CT, D, P, 1>())
-    if (!done && nvb <= 1) {
-      hipLaunchKernelGGL((gdn3_window_kernel<CT, D, P, 1>), dim3(N), dim3(kNT), 0, stream, a);
-      done = true;
-    }
-  if constexpr (win_fits<CT, D, P, V2>())
-    if (!done && nvb <= V2) {
-      hipLaunchKernelGGL((gdn3_window_kernel<CT, D, P, V2>), dim3(N * V2), dim3(kNT), 0, stream, a);
-      done = true;
-    }
-  if constexpr (win_fits<CT, D, P, V4>())
-    if (!done && nvb <= V4) {
-      hipLaunchKernelGGL((gdn3_window_kernel<CT, D, P, V4>), dim3(N * V4), dim3(kNT), 0, stream, a);
-      done = true;
-    }
-  if (!done) hipLaunchKernelGGL((gdn3_window_kernel<CT, D, P, V8>), dim3(N * V8), dim3(kNT), 0, stream, a);
-  return check_launch("gdn3_window_kernel");
-}
-
 template <typename CT, int D, int P>
 int run_gdn3_fwd(G3FwdArgs a, hipStream_t stream) {
   typedef G3D<D> Ge;
@@ -1864,9 +1695,7 @@ int run_gdn3_fwd(G3FwdArgs a, hipStream_t stream) {
     a.live = !first || carried;      // the Kronecker factors may be nonzero
     a.last = c1 == cg1;
     a.complete = (long long)c1 * kSC <= tend && c1 % per == 0;
-    // intervals of several sub-chunks run over batches of them (gdn3_long.hip)
-    rc = c1 - c0 >= 3 ? gdn3_long_interval(a, N, stream) : launch_window<CT, D, P>(a, N, stream);
-    if (rc) return rc;
+    if ((rc = gdn3_long_interval(a, N, stream))) return rc;
     if (a.complete) {
       G3CompactArgs ca{};
       ca.A = a.ab;

@@ -197,7 +197,7 @@ struct G3FwdArgs {
   float* vw;           // [N, P, D] window keys decayed to the window end
   float* gsum;         // [N] log decay since the last compaction
   int c0, c1, first, live, last, complete;
-  // intervals of several sub-chunks (gdn3_long.hip): the copy of the window
+  // intervals (gdn3_long.hip): the copy of the window
   // state the interval leaves (uw / vw themselves, or the other copy), the
   // runs' maps, runs and sub-chunks per run
   float* uw_alt;
@@ -320,7 +320,7 @@ int gdn3_fwd_dispatch(const G3FwdArgs& a, hipStream_t stream);
 bool gdn3_fwd_fused(int D, int P, int Kc, int dtype);
 // bytes of the static scratch of gdnx_gdn3_chunk_fwd_state_noalloc (per device)
 constexpr size_t kG3ScratchBytes = (size_t)64 << 20;
-// workgroups an interval of several sub-chunks is spread over (chains x runs),
+// workgroups an interval is spread over (chains x runs),
 // and what that takes at most beside the state (d = 128, P = 64, 256 chains:
 // the other copy of the window state and the maps of 512 runs)
 constexpr int kG3RunTarget = 512;
@@ -333,7 +333,7 @@ size_t gdn3_workspace_bytes(int N, int D, int P, int dtype);
 // of it, what holds the state between launches (the no-alloc entry's limit
 // counts this part)
 size_t gdn3_state_bytes(int N, int D, int P, int dtype);
-// intervals of several sub-chunks (gdn3_long.hip)
+// the intervals between compactions (gdn3_long.hip)
 size_t gdn3_long_bytes(int N, int D, int P);
 void gdn3_long_carve(G3FwdArgs& a, int N, char* w);
 int gdn3_long_interval(G3FwdArgs& a, int N, hipStream_t stream);

@@ -554,9 +554,15 @@ __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2
 }
 
 // ---------------------------------------------------------------------------
-// dispatch: one workgroup of D/16 waves per chain (each wave 16 value
-// columns), so the chunk's tiles are loaded and the -Wm product formed once
-// per chain and shared through LDS
+// dispatch: a chain's value columns over one workgroup of D/16 waves (each
+// wave 16 columns), which loads and stages the chunk's tiles once, or, while
+// that still gives every workgroup a CU of its own, over two of D/32: a step
+// is bound by what its CU issues and reads from LDS for the waves on it.
+// Forward at d = 128, bf16, 64 chains, T = 8190: 546 us with 8 waves a
+// workgroup, 353 with 4 (500 with 2: the staging of a chunk by two waves takes
+// longer than its products); at 256 chains two workgroups per chain share a
+// CU and are no faster.  (P3 contracts over all value columns: that reverse
+// scan is one workgroup per chain.)
 // ---------------------------------------------------------------------------
 template <typename CT, int D, int C>
 struct ScanCfg {
@@ -565,34 +571,37 @@ struct ScanCfg {
                     sizeof(ScanBwdSmem<CT, D, C, NWV, false>) <= 160 * 1024 &&
                     (sizeof(CT) != 2 || C != 32 || sizeof(ScanBwdSmem<CT, D, C, NWV, true>) <= 160 * 1024),
                 "scan LDS budget");
+  // the chunks that training and inference default to are also built split
+  static constexpr bool SPLIT = NWV > 4 && C == (sizeof(CT) == 2 ? 32 : 16);
 };
+constexpr int kSplitChains = 128;   // chains whose two workgroups each have one of the 256 CUs
 
-template <typename CT, int D, int C>
+template <typename CT, int D, int C, int NWV = D / 16>
 static int launch_scan_fwd(const DeltaArgs& a, hipStream_t stream) {
-  constexpr int NWV = ScanCfg<CT, D, C>::NWV;
   typedef ScanDims<CT, D, C, NWV> Sd;
+  const int nc = a.B * a.H * a.M;
+  if constexpr (ScanCfg<CT, D, C>::SPLIT && NWV > 4)
+    if (nc <= kSplitChains) return launch_scan_fwd<CT, D, C, NWV / 2>(a, stream);
   if (a.chunk_states)
-    hipLaunchKernelGGL((delta_scan_fwd_kernel<CT, D, C, NWV, true>), dim3(a.B * a.H * a.M * Sd::NVB), dim3(Sd::NT),
-                       0, stream, a);
+    hipLaunchKernelGGL((delta_scan_fwd_kernel<CT, D, C, NWV, true>), dim3(nc * Sd::NVB), dim3(Sd::NT), 0, stream, a);
   else
-    hipLaunchKernelGGL((delta_scan_fwd_kernel<CT, D, C, NWV, false>), dim3(a.B * a.H * a.M * Sd::NVB), dim3(Sd::NT),
-                       0, stream, a);
+    hipLaunchKernelGGL((delta_scan_fwd_kernel<CT, D, C, NWV, false>), dim3(nc * Sd::NVB), dim3(Sd::NT), 0, stream, a);
   return check_launch("delta_scan_fwd_kernel");
 }
 
-template <typename CT, int D, int C>
+template <typename CT, int D, int C, int NWV = D / 16>
 static int launch_scan_bwd(const DeltaBwdArgs& a, hipStream_t stream) {
-  constexpr int NWV = ScanCfg<CT, D, C>::NWV;
   typedef ScanDims<CT, D, C, NWV> Sd;
-  if constexpr (sizeof(CT) == 2 && C == 32) {
+  const int nc = a.B * a.H * a.M;
+  if constexpr (sizeof(CT) == 2 && C == 32 && Sd::NVB == 1) {
     if (a.cps > 1) {   // checkpointed form: P3 tiles for delta_grad_seg_kernel
-      hipLaunchKernelGGL((delta_scan_bwd_kernel<CT, D, C, NWV, true>), dim3(a.B * a.H * a.M * Sd::NVB), dim3(Sd::NT),
-                         0, stream, a);
+      hipLaunchKernelGGL((delta_scan_bwd_kernel<CT, D, C, NWV, true>), dim3(nc), dim3(Sd::NT), 0, stream, a);
       return check_launch("delta_scan_bwd_kernel");
     }
   }
-  hipLaunchKernelGGL((delta_scan_bwd_kernel<CT, D, C, NWV, false>), dim3(a.B * a.H * a.M * Sd::NVB), dim3(Sd::NT), 0,
-                     stream, a);
+  if constexpr (ScanCfg<CT, D, C>::SPLIT && NWV > 4)
+    if (nc <= kSplitChains) return launch_scan_bwd<CT, D, C, NWV / 2>(a, stream);
+  hipLaunchKernelGGL((delta_scan_bwd_kernel<CT, D, C, NWV, false>), dim3(nc * Sd::NVB), dim3(Sd::NT), 0, stream, a);
   return check_launch("delta_scan_bwd_kernel");
 }
 

@@ -51,7 +51,7 @@ constexpr int kRes = 2;       // lanes whose states are resident at a time
 template <int D>
 struct SegDims {
   static constexpr int C = 32;                           // sub-chunk (tokens)
-  static constexpr int NSUB = kSegTokens / C;            // sub-chunks per segment
+  static constexpr int NSUB = kSegTokens / C;            // sub-chunks per segment, at most (p.cps)
   static constexpr int NW = D / 16;                      // waves; wave w owns key (and value) tile w
   static constexpr int NT = 64 * NW;
   static constexpr int NDT = D / 16;
@@ -182,8 +182,8 @@ delta_grad_seg_kernel(DeltaBwdArgs p) {
   const int BH = p.B * p.H, M = p.M;
   const int s = blockIdx.x / BH, bh = blockIdx.x % BH, b = bh / p.H, h = bh % p.H;
   const int N = BH * M;
-  const int t_seg = s * kSegTokens;
-  const int nsub = min(Sd::NSUB, (p.T - t_seg + C - 1) / C);
+  const int seg = p.cps * C, t_seg = s * seg;   // tokens per segment
+  const int nsub = min(p.cps, (p.T - t_seg + C - 1) / C);
   // the scans' chunk, which is the stash's record length and the sub-chunk
   // (dispatch rejects any other p.C), so record offsets are shifts
   constexpr int CS = C;
@@ -196,7 +196,7 @@ delta_grad_seg_kernel(DeltaBwdArgs p) {
   const float* k3st = (const float*)(p3st + sg.tiles);   // k.P3 per token
   // this workgroup's float32 carry of the dq, dk, dv sums from one lane pair
   // to the next, [3][sub-chunk][wave][token tile][64 lanes][4]
-  const int NSEG = (p.T + kSegTokens - 1) / kSegTokens;
+  const int NSEG = (p.T + seg - 1) / seg;
   float* const dqs = (float*)((char*)p.ds_stash + delta_seg_carry_offset(N, p.T, D, CS, p.cps)) +
                      ((size_t)bh * NSEG + s) * 3 * kSegTokens * D;
   float* const dks = dqs + kSegTokens * D;
@@ -673,7 +673,8 @@ delta_grad_seg_kernel(DeltaBwdArgs p) {
 }  // namespace
 
 int delta_grad_seg_dispatch(const DeltaBwdArgs& a, hipStream_t stream) {
-  const int NSEG = (a.T + kSegTokens - 1) / kSegTokens;
+  if (a.cps < 1 || a.cps > SegDims<128>::NSUB) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: segment of %d chunks", a.cps);
+  const int seg = a.cps * a.C, NSEG = (a.T + seg - 1) / seg;
   const unsigned grid = (unsigned)(a.B * a.H * NSEG);
   if (a.M > kLaneCap) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: at most %d lanes per head", kLaneCap);
   if (a.C != SegDims<128>::C) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: %d-token chunks only", SegDims<128>::C);

@@ -30,8 +30,8 @@ int delta_chunk_size(int D, int dtype) {
 }
 
 // chunk used when the forward stashes states for the backward: 32 for bf16
-// (with at most 4 lanes per head the stash keeps one state per 256-token
-// segment and the backward recomputes the rest), 16 for float32.  The
+// (with at most 4 lanes per head the stash keeps one state per segment of
+// up to 256 tokens and the backward recomputes the rest), 16 for float32.  The
 // 64-token bf16 chunk stays selectable in the per-chunk stash form: its
 // scans hold one chunk's tiles in LDS instead of two (no overlap of the next
 // chunk's staging), spill registers, and measured 1.5-2x slower on the
@@ -42,9 +42,9 @@ int delta_train_chunk_size(int D, int dtype) {
 }
 
 size_t delta_bwd_workspace_bytes(int B, int T, int H, int M, int D, int C, int dtype) {
-  const int cps = delta_stash_cps(D, C, dtype, M);
+  const int cps = delta_stash_cps(D, C, dtype, M, B * H, T);
   if (cps > 1) {   // see delta_seg_carry_offset
-    const size_t nseg = (size_t)((T + kSegTokens - 1) / kSegTokens);
+    const size_t seg = (size_t)cps * C, nseg = ((size_t)T + seg - 1) / seg;
     return delta_seg_carry_offset(B * H * M, T, D, C, cps) +
            (M > 2 ? 3 * (size_t)B * H * nseg * kSegTokens * D * sizeof(float) : 0);
   }
@@ -116,7 +116,7 @@ extern "C" long long gdnx_delta_chunk_states_bytes(int B, int T, int H, int M, i
   if (C == 0 || !valid_chunk(head_dim, dtype, C) || B < 1 || T < 0 || H < 1 || M < 1 ||
       (head_dim != 64 && head_dim != 128) || !query_sizes_ok(B, T, H, M))
     return -1;
-  const int cps = delta_stash_cps(head_dim, C, dtype, M);
+  const int cps = delta_stash_cps(head_dim, C, dtype, M, B * H, T);
   return (long long)(delta_stash_bytes(B * H * M, T, head_dim, C, dtype, cps) +
                      delta_prep_bytes(B * H * M, T, C, dtype));
 }
@@ -145,7 +145,7 @@ static int fwd_common(const void* q, const void* k, const void* v, const float* 
   if (!valid_chunk(head_dim, dtype, C)) return set_error(GDNX_ERR_SHAPE, "chunk %d invalid for this dtype", chunk);
   if (T == 0) return GDNX_OK;
   DeltaArgs a{q, k, v, a_e, a_w, log_g, state0, y, state_out, chunk_states, B, T, H, M, head_dim, C, dtype,
-              r_norm, workspace, delta_stash_cps(head_dim, C, dtype, M)};
+              r_norm, workspace, delta_stash_cps(head_dim, C, dtype, M, B * H, T)};
   if ((rc = delta_fwd_dispatch(a, (hipStream_t)stream))) return rc;
   const size_t rows = (size_t)B * T * H * M, D = head_dim;
   const FiniteBuf outs[] = {{y, rows * D, dtype}, {state_out, (size_t)B * H * M * D * D, GDNX_DTYPE_F32},
@@ -217,7 +217,7 @@ static int bwd_common(const void* q, const void* k, const void* v, const float* 
   if (T == 0) return GDNX_OK;
   DeltaBwdArgs a{q,  k,  v,  a_e,  a_w,  log_g, dy,      dstate_out, chunk_states, workspace, dq, dk,
                  dv, da_e, da_w, dlog_g, dstate0, B, T, H, M, head_dim, C, dtype,
-                 delta_stash_cps(head_dim, C, dtype, M)};
+                 delta_stash_cps(head_dim, C, dtype, M, B * H, T)};
   if ((rc = delta_bwd_dispatch(a, stages, (hipStream_t)stream))) return rc;
   const size_t rows = (size_t)B * T * H * M, D = head_dim, tok = (size_t)B * T * H * D;
   const bool g = (stages & 2) != 0;

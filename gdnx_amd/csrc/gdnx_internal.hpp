@@ -348,19 +348,26 @@ int delta_prep_dispatch(const DeltaArgs& a, hipStream_t stream);
 int delta_scan_fwd_dispatch(const DeltaArgs& a, hipStream_t stream);
 int delta_scan_bwd_dispatch(const DeltaBwdArgs& a, hipStream_t stream);
 size_t delta_prep_bytes(int nchains, int T, int C, int dtype);
-// Tokens per recompute segment of the checkpointed backward: the forward
-// keeps the state entering every segment, the reverse scan the state
-// gradient leaving it, and the gradient kernel rebuilds the states and state
-// gradients in between.
+// Tokens per recompute segment of the checkpointed backward, at most: the
+// forward keeps the state entering every segment, the reverse scan the state
+// gradient leaving it, and the gradient kernel rebuilds the states in between.
 constexpr int kSegTokens = 256;
 // Chunks per stashed state record: 1 (the state entering every chunk and the
 // state gradient leaving it, read by delta_bwd_grads_kernel) or, for bf16 IO
 // with 32-token chunks and at most 4 lanes per head, one record per
-// kSegTokens-token segment (read by delta_grad_seg_kernel, which recomputes
+// segment (read by delta_grad_seg_kernel, which recomputes
 // the rest in 32-token sub-chunks: the reverse scan's P3 = R dS^T is taken
 // at its chunk ends, so its chunk must be the sub-chunk).
-__host__ __device__ inline int delta_stash_cps(int D, int C, int dtype, int M) {
-  return (dtype == GDNX_DTYPE_BF16 && C == 32 && M >= 1 && M <= 4 && (D == 64 || D == 128)) ? kSegTokens / C : 1;
+// The gradient kernel runs one workgroup per (b, h, segment) and one to a CU,
+// each walking its segment's sub-chunks in order; so segments of 256 tokens
+// (the least state traffic) are halved while they leave CUs without a
+// workgroup, down to 64 tokens.  BH = 16, T = 1999, 4 lanes, d = 128: 172 us
+// with 128 workgroups of 256 tokens, 112 with 256 of 128.
+__host__ __device__ inline int delta_stash_cps(int D, int C, int dtype, int M, int BH, int T) {
+  if (!(dtype == GDNX_DTYPE_BF16 && C == 32 && M >= 1 && M <= 4 && (D == 64 || D == 128))) return 1;
+  int cps = kSegTokens / C;
+  while (cps > 2 && (long long)BH * ((T + (long long)cps * C - 1) / ((long long)cps * C)) < 256) cps /= 2;
+  return cps;
 }
 // Per-chain stash geometry: NC chunks; a state record every cps chunks.
 struct StashGeom {

@@ -58,6 +58,8 @@ SIGNATURES = {
     "gdnx_gdn3_train_states_bytes": (_c_ll, [_c_int] * 7),
     "gdnx_gdn3_chunk_bwd": (_c_int, [_vp] * 3 + [_c_int] + [_vp] * 2 + [_c_int] + [_vp] * 9
                             + [_c_int] * 13 + [_vp]),
+    "gdnx_gdn3_chunk_bwd_io": (_c_int, [_vp] * 3 + [_c_int] + [_vp] * 2 + [_c_int] + [_vp] * 9
+                               + [_c_int] * 13 + [_vp]),
     "gdnx_gdn3_compact": (_c_int, [_vp] * 8 + [_c_int] * 8 + [_c_float, _c_int, _vp]),
     "gdnx_kron_read": (_c_int, [_vp] * 6 + [_c_int] * 9 + [_vp]),
     "gdnx_gdn3_coeff": (_c_int, [_vp] * 3 + [_c_int] * 6 + [_vp]),
@@ -69,6 +71,7 @@ SIGNATURES = {
     "gdnx_gdn3_lane_rope_pairs": (_c_int, [_c_int, _c_int, _vp]),
     "gdnx_gdn3_prologue_fwd": (_c_int, [_vp] * 15 + [_c_int] * 6 + [_c_float, _c_int, _vp]),
     "gdnx_gdn3_prologue_bwd": (_c_int, [_vp] * 20 + [_c_int] * 6 + [_c_float, _c_int, _vp]),
+    "gdnx_gdn3_prologue_bwd_io": (_c_int, [_vp] * 20 + [_c_int] * 6 + [_c_float, _c_int, _vp]),
     "gdnx_gdn3_epilogue_fwd": (_c_int, [_vp] * 4 + [_c_int] * 6 + [_vp]),
     "gdnx_gdn3_epilogue_workspace_bytes": (_c_ll, [_c_int] * 4),
     "gdnx_gdn3_epilogue_bwd": (_c_int, [_vp] * 8 + [_c_int] * 6 + [_vp]),

@@ -663,12 +663,13 @@ extern "C" int gdnx_gdn3_decode_step(const void* q, const void* k, const void* v
   return finite_outputs(outs, 2, (hipStream_t)stream);
 }
 
-extern "C" int gdnx_gdn3_chunk_bwd(const void* q, const void* k, const void* v, int qkv_lanes,
-                                   const float* b_gates, const float* w_gates, int gate_channels,
-                                   const float* decay, const void* dy, const void* train_states, float* dq,
-                                   float* dk, float* dv, float* db_gates, float* dw_gates, float* ddecay, int B,
-                                   int T, int H, int M, int head_dim, int R, int P, int compact_every, int a_v,
-                                   int a_k, int b_v, int b_k, int dtype, void* stream) {
+static int g3_chunk_bwd(const void* q, const void* k, const void* v, int qkv_lanes,
+                        const float* b_gates, const float* w_gates, int gate_channels,
+                        const float* decay, const void* dy, const void* train_states, void* dq,
+                        void* dk, void* dv, float* db_gates, float* dw_gates, float* ddecay, int B,
+                        int T, int H, int M, int head_dim, int R, int P, int compact_every, int a_v,
+                        int a_k, int b_v, int b_k, int dtype, int grad_io,
+                        void* stream) {
   g_err[0] = 0;
   int rc = check_common(q, k, v, B, T, H, M, head_dim, dtype);
   if (rc) return rc;
@@ -692,13 +693,33 @@ extern "C" int gdnx_gdn3_chunk_bwd(const void* q, const void* k, const void* v, 
                      "16-byte aligned");
   if (T == 0) return GDNX_OK;
   G3BwdArgs a{q, k, v, b_gates, w_gates, decay, dy, train_states, dq, dk, dv, db_gates, dw_gates, ddecay,
-              B, T, H, M, head_dim, P, compact_every, qkv_lanes, gate_channels, dtype};
+              B, T, H, M, head_dim, P, compact_every, qkv_lanes, gate_channels, dtype, grad_io};
   if ((rc = gdn3_bwd_dispatch(a, (hipStream_t)stream))) return rc;
   const size_t rows = (size_t)B * T * H * M;
-  const FiniteBuf outs[] = {{dq, rows * head_dim, GDNX_DTYPE_F32}, {dk, rows * head_dim, GDNX_DTYPE_F32},
-                            {dv, rows * head_dim, GDNX_DTYPE_F32}, {db_gates, rows * gate_channels, GDNX_DTYPE_F32},
-                            {dw_gates, rows * gate_channels, GDNX_DTYPE_F32}, {ddecay, rows, GDNX_DTYPE_F32}};
+  const int gd = grad_io ? dtype : GDNX_DTYPE_F32;
+  const FiniteBuf outs[] = {{dq, rows * head_dim, gd}, {dk, rows * head_dim, gd}, {dv, rows * head_dim, gd},
+                            {db_gates, rows * gate_channels, GDNX_DTYPE_F32}, {dw_gates, rows * gate_channels, GDNX_DTYPE_F32}, {ddecay, rows, GDNX_DTYPE_F32}};
   return finite_outputs(outs, 6, (hipStream_t)stream);
+}
+
+extern "C" int gdnx_gdn3_chunk_bwd(const void* q, const void* k, const void* v, int qkv_lanes,
+                                   const float* b_gates, const float* w_gates, int gate_channels,
+                                   const float* decay, const void* dy, const void* train_states, float* dq,
+                                   float* dk, float* dv, float* db_gates, float* dw_gates, float* ddecay, int B,
+                                   int T, int H, int M, int head_dim, int R, int P, int compact_every, int a_v,
+                                   int a_k, int b_v, int b_k, int dtype, void* stream) {
+  return g3_chunk_bwd(q, k, v, qkv_lanes, b_gates, w_gates, gate_channels, decay, dy, train_states, dq, dk, dv,
+                      db_gates, dw_gates, ddecay, B, T, H, M, head_dim, R, P, compact_every, a_v, a_k, b_v, b_k, dtype, 0, stream);
+}
+
+extern "C" int gdnx_gdn3_chunk_bwd_io(const void* q, const void* k, const void* v, int qkv_lanes,
+                                      const float* b_gates, const float* w_gates, int gate_channels,
+                                      const float* decay, const void* dy, const void* train_states, void* dq,
+                                      void* dk, void* dv, float* db_gates, float* dw_gates, float* ddecay, int B,
+                                      int T, int H, int M, int head_dim, int R, int P, int compact_every, int a_v,
+                                      int a_k, int b_v, int b_k, int dtype, void* stream) {
+  return g3_chunk_bwd(q, k, v, qkv_lanes, b_gates, w_gates, gate_channels, decay, dy, train_states, dq, dk, dv,
+                      db_gates, dw_gates, ddecay, B, T, H, M, head_dim, R, P, compact_every, a_v, a_k, b_v, b_k, dtype, 1, stream);
 }
 
 extern "C" int gdnx_gdn3_compact(const float* A, const float* Bf, const float* U, const float* Vb,
@@ -912,14 +933,14 @@ extern "C" int gdnx_gdn3_prologue_fwd(const void* q, const void* k, const void* 
   return gdn3_prologue_dispatch(a, false, dtype, (hipStream_t)stream);
 }
 
-extern "C" int gdnx_gdn3_prologue_bwd(const void* b_proj, const void* proj_a, const void* w_proj,
-                                      const void* proj_b, const void* decay_proj, const float* rates,
-                                      const float* rope_cos, const float* rope_sin, const float* d_q_rope,
-                                      const float* d_k_rope, const float* d_b_gates, const float* d_w_gates,
-                                      const float* d_decay, float* dq, float* dk, float* d_b_proj,
-                                      float* d_proj_a, float* d_w_proj, float* d_proj_b, float* d_decay_proj,
-                                      int B, int T, int H, int M, int key_dim, int value_dim, float decay_clamp,
-                                      int dtype, void* stream) {
+static int g3_prologue_bwd(const void* b_proj, const void* proj_a, const void* w_proj,
+                           const void* proj_b, const void* decay_proj, const float* rates,
+                           const float* rope_cos, const float* rope_sin, const void* d_q_rope,
+                           const void* d_k_rope, const float* d_b_gates, const float* d_w_gates,
+                           const float* d_decay, void* dq, void* dk, void* d_b_proj,
+                           void* d_proj_a, void* d_w_proj, void* d_proj_b, void* d_decay_proj,
+                           int B, int T, int H, int M, int key_dim, int value_dim, float decay_clamp,
+                           int dtype, int grad_io, void* stream) {
   g_err[0] = 0;
   int rc = layer_sizes(B, T, H, M, key_dim, value_dim, dtype, true);
   if (rc != GDNX_OK) return rc;
@@ -933,10 +954,37 @@ extern "C" int gdnx_gdn3_prologue_bwd(const void* b_proj, const void* proj_a, co
   a.dqr = d_q_rope; a.dkr = d_k_rope; a.dbg = d_b_gates; a.dwg = d_w_gates; a.ddec = d_decay;
   a.dq = dq; a.dk = dk; a.dbp = d_b_proj; a.dpa = d_proj_a; a.dwp = d_w_proj; a.dpb = d_proj_b;
   a.ddp = d_decay_proj;
+  a.grad_io = grad_io;
   a.rows = (long long)B * T * H;
   a.T = T; a.H = H; a.M = M; a.K = key_dim; a.V = value_dim; a.clamp = decay_clamp;
   gdn3_lane_pairs(M, key_dim, a.pairs);
   return gdn3_prologue_dispatch(a, true, dtype, (hipStream_t)stream);
+}
+
+extern "C" int gdnx_gdn3_prologue_bwd(const void* b_proj, const void* proj_a, const void* w_proj,
+                                      const void* proj_b, const void* decay_proj, const float* rates,
+                                      const float* rope_cos, const float* rope_sin, const float* d_q_rope,
+                                      const float* d_k_rope, const float* d_b_gates, const float* d_w_gates,
+                                      const float* d_decay, float* dq, float* dk, float* d_b_proj,
+                                      float* d_proj_a, float* d_w_proj, float* d_proj_b, float* d_decay_proj,
+                                      int B, int T, int H, int M, int key_dim, int value_dim, float decay_clamp,
+                                      int dtype, void* stream) {
+  return g3_prologue_bwd(b_proj, proj_a, w_proj, proj_b, decay_proj, rates, rope_cos, rope_sin, d_q_rope, d_k_rope, d_b_gates,
+                         d_w_gates, d_decay, dq, dk, d_b_proj, d_proj_a, d_w_proj, d_proj_b, d_decay_proj, B, T, H, M,
+                         key_dim, value_dim, decay_clamp, dtype, 0, stream);
+}
+
+extern "C" int gdnx_gdn3_prologue_bwd_io(const void* b_proj, const void* proj_a, const void* w_proj,
+                                         const void* proj_b, const void* decay_proj, const float* rates,
+                                         const float* rope_cos, const float* rope_sin, const void* d_q_rope,
+                                         const void* d_k_rope, const float* d_b_gates, const float* d_w_gates,
+                                         const float* d_decay, void* dq, void* dk, void* d_b_proj,
+                                         void* d_proj_a, void* d_w_proj, void* d_proj_b, void* d_decay_proj,
+                                         int B, int T, int H, int M, int key_dim, int value_dim, float decay_clamp,
+                                         int dtype, void* stream) {
+  return g3_prologue_bwd(b_proj, proj_a, w_proj, proj_b, decay_proj, rates, rope_cos, rope_sin, d_q_rope, d_k_rope, d_b_gates,
+                         d_w_gates, d_decay, dq, dk, d_b_proj, d_proj_a, d_w_proj, d_proj_b, d_decay_proj, B, T, H, M,
+                         key_dim, value_dim, decay_clamp, dtype, 1, stream);
 }
 
 extern "C" long long gdnx_gdn3_epilogue_workspace_bytes(int B, int T, int H, int value_dim) {

@@ -248,13 +248,13 @@ struct G3BwdArgs {
   const float* dec;
   const void* dy;             // [B,T,H,M,D] compute dtype
   const void* train_states;   // the forward's stash (layout G3Stash)
-  float* dq;                  // [B,T,H,M,D] per lane
-  float* dk;
-  float* dv;
+  void* dq;                   // [B,T,H,M,D] per lane, float32 (grad_io: the IO type)
+  void* dk;
+  void* dv;
   float* dbg;                 // gate layout ([.., D] or [..])
   float* dwg;
   float* ddec;                // [B,T,H,M]
-  int B, T, H, M, D, P, Kc, qkv_lanes, gate_ch, dtype;
+  int B, T, H, M, D, P, Kc, qkv_lanes, gate_ch, dtype, grad_io;
 };
 
 struct KronReadArgs {
@@ -284,18 +284,19 @@ struct G3ProArgs {
   float* bg;
   float* wg;
   float* dec;       // [rows, M]
-  const float* dqr; // backward inputs, float32, forward-output layouts
-  const float* dkr;
+  const void* dqr;  // backward inputs, float32 (grad_io: dqr, dkr in the IO type), forward-output layouts
+  const void* dkr;
   const float* dbg;
   const float* dwg;
   const float* ddec;
-  float* dq;        // backward outputs, float32, forward-input layouts
-  float* dk;
-  float* dbp;
-  float* dpa;
-  float* dwp;
-  float* dpb;
-  float* ddp;
+  void* dq;         // backward outputs, float32 (grad_io: the IO type), forward-input layouts
+  void* dk;
+  void* dbp;
+  void* dpa;
+  void* dwp;
+  void* dpb;
+  void* ddp;
+  int grad_io;
   long long rows;
   int T, H, M, K, V;
   int pairs[4];

@@ -153,12 +153,13 @@ class _GDN3Chunk(torch.autograd.Function):
         M, R, P, factors, _, Kc, _ = ctx.cfg
         if dy is None:
             return (None,) * 9
+        # per-lane q, k, v: their gradients in the IO dtype as they are written
         dq, dk, dv, db, dw, ddec = ops.gdn3_chunk_bwd(q, k, v, bg, wg, dec, dy, tst, M=M, R=R, P=P,
-                                                      factors=factors, compact_every=Kc)
+                                                      factors=factors, compact_every=Kc, io_grads=q.dim() == 5)
         if q.dim() == 4:   # q, k, v shared by the lanes: their lane sums, in the IO dtype
             return (ops.lane_sum(dq, q.dtype), ops.lane_sum(dk, k.dtype), ops.lane_sum(dv, v.dtype), db, dw,
                     ddec, None, None, None)
-        return dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), db, dw, ddec, None, None, None
+        return dq, dk, dv, db, dw, ddec, None, None, None
 
 
 def gdn3_recurrent_state(q, k, v, b_gates, w_gates, decay_factors, *, R=4, P=16,

@@ -94,7 +94,8 @@ class _Prologue(torch.autograd.Function):
             return torch.zeros(shape, dtype=torch.float32, device=bp.device) if t is None else t
         grads = ops.gdn3_prologue_bwd(bp, pa, wp, pb, dp, rates, cos, sin, g(dqr, (B, T, H, M, K)),
                                       g(dkr, (B, T, H, M, K)), g(dbg, (B, T, H, M, K)), g(dwg, (B, T, H, M, V)),
-                                      g(ddec, (B, T, H, M)), ctx.decay_clamp)
+                                      g(ddec, (B, T, H, M)), ctx.decay_clamp,
+                                      io_grads=all(d == bp.dtype for d in ctx.in_dtypes))
         dq, dk, dbp, dpa, dwp, dpb, ddp = grads
         out = [t.to(d) for t, d in zip((dq, dk, dbp, dpa, dwp, dpb, ddp), ctx.in_dtypes)]
         return (*out, None, None)

@@ -705,10 +705,11 @@ def gdn3_decode_step(q, k, v, b_gates, w_gates, decay, sketch, state, pos, *, R=
 
 
 def gdn3_chunk_bwd(q, k, v, b_gates, w_gates, decay, dy, train_states, *, M, R=4, P=16,
-                   factors=(16, 16, 8, 8), compact_every=None):
+                   factors=(16, 16, 8, 8), compact_every=None, io_grads=False):
     """Backward of gdn3_chunk_fwd (gdnx_gdn3_chunk_bwd) from the stash its
     save_states call returned.  Returns float32 (dq, dk, dv [B,T,H,M,D] per
-    lane, db_gates, dw_gates in the gates' layout, ddecay [B,T,H,M])."""
+    lane, db_gates, dw_gates in the gates' layout, ddecay [B,T,H,M]); with
+    io_grads, dq, dk and dv in q's dtype (gdnx_gdn3_chunk_bwd_io)."""
     lib = _lib.load()
     a_v, a_k, b_v, b_k = factors
     B, T, H = q.shape[:3]
@@ -718,15 +719,16 @@ def gdn3_chunk_bwd(q, k, v, b_gates, w_gates, decay, dy, train_states, *, M, R=4
     Kc = P if compact_every is None else int(compact_every)
     dy = dy.to(q.dtype).contiguous()
     _need(tuple(dy.shape) == (B, T, H, M, D), "dy must be [B,T,H,M,D]")
-    dq, dk, dv = (torch.empty(B, T, H, M, D, dtype=torch.float32, device=q.device) for _ in range(3))
+    gdt = q.dtype if io_grads else torch.float32
+    dq, dk, dv = (torch.empty(B, T, H, M, D, dtype=gdt, device=q.device) for _ in range(3))
     db, dw = torch.empty_like(b_gates), torch.empty_like(w_gates)
     ddec = torch.empty_like(decay)
     with torch.cuda.device(q.device):
-        rc = lib.gdnx_gdn3_chunk_bwd(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), lanes, _lib.ptr(b_gates),
-                                     _lib.ptr(w_gates), gate_ch, _lib.ptr(decay), _lib.ptr(dy),
-                                     _lib.ptr(train_states), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(db),
-                                     _lib.ptr(dw), _lib.ptr(ddec), B, T, H, M, D, R, P, Kc, a_v, a_k, b_v, b_k,
-                                     _lib.dtype_code(q.dtype), _lib.stream_of(q))
+        fn = lib.gdnx_gdn3_chunk_bwd_io if io_grads else lib.gdnx_gdn3_chunk_bwd
+        rc = fn(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), lanes, _lib.ptr(b_gates), _lib.ptr(w_gates), gate_ch,
+                _lib.ptr(decay), _lib.ptr(dy), _lib.ptr(train_states), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv),
+                _lib.ptr(db), _lib.ptr(dw), _lib.ptr(ddec), B, T, H, M, D, R, P, Kc, a_v, a_k, b_v, b_k,
+                _lib.dtype_code(q.dtype), _lib.stream_of(q))
     _lib.check(rc, "gdnx_gdn3_chunk_bwd")
     return dq, dk, dv, db, dw, ddec
 
@@ -806,30 +808,33 @@ def gdn3_prologue_fwd(q, k, b_proj, proj_a, w_proj, proj_b, decay_proj, rates, r
 
 
 def gdn3_prologue_bwd(b_proj, proj_a, w_proj, proj_b, decay_proj, rates, rope_cos, rope_sin,
-                      d_q_rope, d_k_rope, d_b_gates, d_w_gates, d_decay, decay_clamp=0.999):
+                      d_q_rope, d_k_rope, d_b_gates, d_w_gates, d_decay, decay_clamp=0.999, io_grads=False):
     """Backward of gdn3_prologue_fwd; the IO inputs in the forward's compute
     dtype.  Returns float32 (dq, dk [B,T,H,K], d_b_proj, d_proj_a, d_w_proj,
-    d_proj_b, d_decay_proj)."""
+    d_proj_b, d_decay_proj); with io_grads d_q_rope and d_k_rope are taken and
+    the results given in the compute dtype (gdnx_gdn3_prologue_bwd_io)."""
     lib = _lib.load()
     B, T, H, M, K = b_proj.shape
     V = w_proj.shape[-1]
     dev = b_proj.device
-    f32 = [t.float().contiguous() for t in (d_q_rope, d_k_rope, d_b_gates, d_w_gates, d_decay)]
-    _need(tuple(f32[0].shape) == tuple(f32[1].shape) == (B, T, H, M, K), "d_q_rope / d_k_rope must be [B,T,H,M,K]")
-    _need(tuple(f32[2].shape) == (B, T, H, M, K) and tuple(f32[3].shape) == (B, T, H, M, V)
-          and tuple(f32[4].shape) == (B, T, H, M), "bad gate / decay gradient shapes")
-    dq = torch.empty(B, T, H, K, dtype=torch.float32, device=dev)
+    gdt = b_proj.dtype if io_grads else torch.float32
+    grads = [t.to(gdt).contiguous() for t in (d_q_rope, d_k_rope)]
+    grads += [t.float().contiguous() for t in (d_b_gates, d_w_gates, d_decay)]
+    _need(tuple(grads[0].shape) == tuple(grads[1].shape) == (B, T, H, M, K), "d_q_rope / d_k_rope must be [B,T,H,M,K]")
+    _need(tuple(grads[2].shape) == (B, T, H, M, K) and tuple(grads[3].shape) == (B, T, H, M, V)
+          and tuple(grads[4].shape) == (B, T, H, M), "bad gate / decay gradient shapes")
+    dq = torch.empty(B, T, H, K, dtype=gdt, device=dev)
     dk = torch.empty_like(dq)
-    dbp = torch.empty(B, T, H, M, K, dtype=torch.float32, device=dev)
-    dwp = torch.empty(B, T, H, M, V, dtype=torch.float32, device=dev)
-    dpa = torch.empty(B, T, H, dtype=torch.float32, device=dev)
+    dbp = torch.empty(B, T, H, M, K, dtype=gdt, device=dev)
+    dwp = torch.empty(B, T, H, M, V, dtype=gdt, device=dev)
+    dpa = torch.empty(B, T, H, dtype=gdt, device=dev)
     dpb = torch.empty_like(dpa)
-    ddp = torch.empty(B, T, H, M, 4, dtype=torch.float32, device=dev)
+    ddp = torch.empty(B, T, H, M, 4, dtype=gdt, device=dev)
     with torch.cuda.device(dev):
-        rc = lib.gdnx_gdn3_prologue_bwd(*map(_lib.ptr, (b_proj, proj_a, w_proj, proj_b, decay_proj, rates, rope_cos,
-                                                        rope_sin, *f32, dq, dk, dbp, dpa, dwp, dpb, ddp)),
-                                        B, T, H, M, K, V, float(decay_clamp), _lib.dtype_code(b_proj.dtype),
-                                        _lib.stream_of(b_proj))
+        fn = lib.gdnx_gdn3_prologue_bwd_io if io_grads else lib.gdnx_gdn3_prologue_bwd
+        rc = fn(*map(_lib.ptr, (b_proj, proj_a, w_proj, proj_b, decay_proj, rates, rope_cos, rope_sin, *grads, dq, dk,
+                                dbp, dpa, dwp, dpb, ddp)),
+                B, T, H, M, K, V, float(decay_clamp), _lib.dtype_code(b_proj.dtype), _lib.stream_of(b_proj))
     _lib.check(rc, "gdnx_gdn3_prologue_bwd")
     return dq, dk, dbp, dpa, dwp, dpb, ddp
 

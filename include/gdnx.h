@@ -72,15 +72,15 @@ int gdnx_delta_train_chunk_size(int head_dim, int dtype);
  * C x C compute-dtype matrices, and four float32 per-token factors), which
  * the backward's reverse scan reuses.  The states are the one entering every
  * chunk, except for bf16 IO with 32-token chunks and at most 4 lanes per head
- * (the training default): there only the state entering every 256-token
- * segment is kept, and the backward recomputes the others from the net
+ * (the training default): there only the state entering every segment
+ * (256 tokens, or 128 or 64 while those leave CUs idle) is kept, and the backward recomputes the others from the net
  * writes (checkpointed form). */
 long long gdnx_delta_chunk_states_bytes(int B, int T, int H, int M, int head_dim, int chunk,
                                         int dtype);
 
 /* Bytes of the backward's workspace for the given chunk (0 = train default;
  * -1 if invalid, or beyond 2^30 chains or 2^40 token-chains): the state
- * gradients leaving every chunk (every 256-token segment in the checkpointed
+ * gradients leaving every chunk (every segment in the checkpointed
  * form) and dB = T^T dR of every chunk, laid out as the forward's stash; in
  * the checkpointed form then P3 = R dS^T of every chunk (bf16, the gradient
  * kernel's dk tile layout) and k.P3 per token (float32), and with more than
@@ -427,6 +427,15 @@ int gdnx_gdn3_chunk_bwd(const void* q, const void* k, const void* v, int qkv_lan
                         int T, int H, int M, int head_dim, int R, int P, int compact_every, int a_v,
                         int a_k, int b_v, int b_k, int dtype, void* stream);
 
+/* gdnx_gdn3_chunk_bwd with dq, dk, dv in the IO dtype (each value rounded
+ * once), for per-lane q, k, v whose gradients no lane sum follows. */
+int gdnx_gdn3_chunk_bwd_io(const void* q, const void* k, const void* v, int qkv_lanes,
+                        const float* b_gates, const float* w_gates, int gate_channels,
+                        const float* decay, const void* dy, const void* train_states, void* dq,
+                        void* dk, void* dv, float* db_gates, float* dw_gates, float* ddecay, int B,
+                        int T, int H, int M, int head_dim, int R, int P, int compact_every, int a_v,
+                        int a_k, int b_v, int b_k, int dtype, void* stream);
+
 /* Lane sum: out[r][d] = sum over m = 0 .. M-1, in that order, of x[r][m][d]
  * (x float32 [rows][M][D]; out [rows][D] in dtype GDNX_DTYPE_F32 or _BF16;
  * D a multiple of 8, both 16-byte aligned).  The gradient of q, k or v
@@ -505,6 +514,18 @@ int gdnx_gdn3_prologue_bwd(const void* b_proj, const void* proj_a, const void* w
                            const float* d_k_rope, const float* d_b_gates, const float* d_w_gates,
                            const float* d_decay, float* dq, float* dk, float* d_b_proj,
                            float* d_proj_a, float* d_w_proj, float* d_proj_b, float* d_decay_proj,
+                           int B, int T, int H, int M, int key_dim, int value_dim, float decay_clamp,
+                           int dtype, void* stream);
+
+/* gdnx_gdn3_prologue_bwd with d_q_rope, d_k_rope and the input gradients in
+ * `dtype` (float32 arithmetic, each result rounded once; d_b_gates, d_w_gates
+ * and d_decay float32). */
+int gdnx_gdn3_prologue_bwd_io(const void* b_proj, const void* proj_a, const void* w_proj,
+                           const void* proj_b, const void* decay_proj, const float* rates,
+                           const float* rope_cos, const float* rope_sin, const void* d_q_rope,
+                           const void* d_k_rope, const float* d_b_gates, const float* d_w_gates,
+                           const float* d_decay, void* dq, void* dk, void* d_b_proj,
+                           void* d_proj_a, void* d_w_proj, void* d_proj_b, void* d_decay_proj,
                            int B, int T, int H, int M, int key_dim, int value_dim, float decay_clamp,
                            int dtype, void* stream);
 

@@ -636,8 +636,8 @@ def bench_kmd2(args):
         t_fwd, _ = timed(fwd, args.kernel_iters)
         t_bwd, _ = timed(lambda: ops.delta_chan_bwd(q, k, v, be, bw, lg, dy, st["cs"]), args.kernel_iters)
     f_fwd = flops_chan(B, T, H, D)
-    kernels = {"chan_prep_kernel+chan_scan_fwd_kernel": (t_fwd, f_fwd),
-               "chan_scan_bwd_kernel+chan_grads_kernel": (t_bwd, 2 * f_fwd)}
+    kernels = {"chan_prep_kernel+chan_split_fwd_kernel": (t_fwd, f_fwd),
+               "chan_split_bwd_kernel+chan_grads_kernel": (t_bwd, 2 * f_fwd)}
     dom = max(kernels, key=lambda n: kernels[n][0])
     t_dom, f_dom = kernels[dom]
     achieved = f_dom / t_dom / 1e12

@@ -20,9 +20,10 @@
 // the cumulative decay product instead, which is valid only at its chunk of
 // 16 and moderate decays.  Three kernels, as for the scalar decay: the
 // forward state scan, the reverse scan of the state gradient, and the
-// per-chunk gradient kernel.  One workgroup of D/16 waves per chain (scans)
-// or per chunk (gradients); wave w owns value (and, in the gradient kernel,
-// key) columns 16w..16w+15.
+// per-chunk gradient kernel, here with a prep kernel in front that writes the
+// scans' operands chunk by chunk.  One workgroup of D/16 waves per chunk
+// (prep, gradients), wave w owning value (and key) columns 16w..16w+15; the
+// scans' split is described at their kernels.
 #include "delta_common.hpp"
 #include "gdnx_internal.hpp"
 
@@ -137,7 +138,7 @@ __device__ __forceinline__ float chunk_scalar(const float* base, int b, int t0, 
 // per-chunk operand records (state independent, one workgroup per chunk)
 //   forward:  U = T diag(beta_w) V, -Wm = -T diag(beta_e) (K o e^G), Q o e^G,
 //             (K o e^{G_L - G})^T, Aq, e^{G_L}
-//   backward: K o e^{G_L - G}, (Q o e^G)^T, (K o e^G)^T, T^T, Aq^T, beta_e, e^{G_L}
+//   backward: K o e^{G_L - G}, (Q o e^G)^T, -Wm^T, T^T, Aq^T, e^{G_L}
 // so that the scans carry only the state-dependent products.
 // ---------------------------------------------------------------------------
 template <int D>
@@ -145,9 +146,9 @@ struct ChRec {
   static constexpr int CD = CC * D;
   static constexpr int F_U = 0, F_NWM = CD, F_QE = 2 * CD, F_KFT = 3 * CD, F_AQ = 4 * CD, F_EGL = 4 * CD + CC * CC;
   static constexpr int FN = 4 * CD + CC * CC + D;
-  static constexpr int B_KF = 0, B_QET = CD, B_KET = 2 * CD, B_TT = 3 * CD, B_AQT = 3 * CD + CC * CC,
-                       B_BE = 3 * CD + 2 * CC * CC, B_EGL = 3 * CD + 2 * CC * CC + CC;
-  static constexpr int BN = 3 * CD + 2 * CC * CC + CC + D;
+  static constexpr int B_KF = 0, B_QET = CD, B_NWT = 2 * CD, B_TT = 3 * CD, B_AQT = 3 * CD + CC * CC,
+                       B_EGL = 3 * CD + 2 * CC * CC;
+  static constexpr int BN = 3 * CD + 2 * CC * CC + D;
   static_assert(FN % 4 == 0 && BN % 4 == 0 && F_EGL % 4 == 0 && B_EGL % 4 == 0, "16-byte aligned records");
 };
 
@@ -220,6 +221,9 @@ __global__ void __launch_bounds__(64 * (D / 16)) chan_prep_kernel(ChanArgs p) {
     f32x4 acc = zero4();
     mma(acc, ld_frag(&sm.ket[(16 * wave + n16) * LDC], g4), bt);
     *(f32x4*)&fr[Rc::F_NWM + n16 * D + 16 * wave + 4 * g4] = -acc;
+    if constexpr (BWD)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) br[Rc::B_NWT + (16 * wave + 4 * g4 + s) * CC + n16] = -acc[s];
   }
   {  // U = T diag(beta_w) V on value tile wave, stored as rows
     f32x4 acc = zero4();
@@ -231,7 +235,6 @@ __global__ void __launch_bounds__(64 * (D / 16)) chan_prep_kernel(ChanArgs p) {
     fr[Rc::F_KFT + e] = sm.kft[d * LDC + i];
     if constexpr (BWD) {
       br[Rc::B_QET + e] = sm.qet[d * LDC + i];
-      br[Rc::B_KET + e] = sm.ket[d * LDC + i];
     }
   }
   for (int e = tid; e < CC * CC; e += NT) {
@@ -246,253 +249,346 @@ __global__ void __launch_bounds__(64 * (D / 16)) chan_prep_kernel(ChanArgs p) {
     fr[Rc::F_EGL + e] = o.eGL[e];
     if constexpr (BWD) br[Rc::B_EGL + e] = o.eGL[e];
   }
-  if constexpr (BWD)
-    if (tid < CC) br[Rc::B_BE + tid] = o.be[tid];
 }
 
 // ---------------------------------------------------------------------------
-// forward state scan: one workgroup of NWV waves per (chain, block of 16 NWV
-// value columns); per chunk, from the record:
+// The scans, per chunk from the record
 //   R = U - Wm S0,  Y = (Q o e^G) S0 + Aq R,  S = diag(e^{G_L}) S0 + (K o e^{G_L - G})^T R
-// With SCORE (|r_t| requested) a chain's value columns stay in one workgroup.
+// and the reverse below, with a chain's state split over keys as well as
+// values: a workgroup of four waves per (chain, NV tiles of 16 value columns),
+// wave w carrying the D / 4 keys 16 KT w ... of those columns in registers.
+// Per chunk each wave forms its keys' part of Wm S0 (K dS backward); the parts
+// are summed through LDS, and every wave updates its own keys with the sum.
+// No wave reads another's operands, so the records go from memory straight
+// into MFMA fragments, PF chunks ahead, and a step has one barrier.  With few
+// chains a step is bound by its latency: the fp32 MFMAs (16 x 16 x 4, 32
+// cycles) over D / 4 keys, then the exchange.  d = 128: B = 2, T = 512, H = 16
+// with stash, forward / reverse 105 / 90 us with only the value columns split,
+// 43 / 45 us so (49 / 51 us while a step could wait for a later chunk's
+// loads); B = 1, T = 2048 forward 292 us, then 125 us.
 // ---------------------------------------------------------------------------
-template <int D, int NWV>
-struct alignas(16) ChanScanFSmem {
-  static constexpr int LDD = D + 4, BV = 16 * NWV, LDU = BV + 4;
-  float nwm[CC * LDD];
-  float qe[CC * LDD];
-  float kft[D * LDC];
-  float aq[CC * LDC];
-  float egl[D];
-  float u[CC * LDU];
-  float rn[NWV][CC];
+template <int D>
+struct ChSplit {
+  static constexpr int KT = D / 64;   // key tiles per wave
+  static constexpr int NVT = D / 16;  // value tiles
+  // chunks of operands in flight (as the registers of NV value tiles leave room for)
+  static constexpr int PF(int nv, bool score) { return nv == 1 ? 4 : nv == 2 ? (score ? 3 : 4) : 2; }
 };
+// acc0 + acc1 += sum_t A_t B_t: the fp32 MFMAs of a product over all of a
+// wave's key tiles as two chains
+template <int KT>
+__device__ __forceinline__ void mma2(f32x4& acc0, f32x4& acc1, const f32x4 (&a)[KT], const f32x4 (&b)[KT]) {
+#pragma unroll
+  for (int t = 0; t < KT; ++t)
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) {
+      acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][s], b[t][s], acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][s + 1], b[t][s + 1], acc1, 0, 0, 0);
+    }
+}
+// Operands of a record: its resource, a lane's byte offset and the wave's
+// uniform one, in floats (no vector address is formed).
+__device__ __forceinline__ f32x4 rec_load4(__amdgpu_buffer_rsrc_t r, unsigned lane_bytes, int at) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)lane_bytes, at * 4, 0));
+}
+__device__ __forceinline__ float rec_load1(__amdgpu_buffer_rsrc_t r, unsigned lane_bytes, int at) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)lane_bytes, at * 4, 0));
+}
+// Keeps the loads of a chunk's operands together and after the step that read
+// the last ones from the same registers: with the chunks' loads in order, and a
+// loop with one exit, a step waits for its own operands only.
+__device__ __forceinline__ void load_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+template <int NV>
+struct alignas(16) ChanExchange {
+  f32x4 r[2][NV][4][64];   // the waves' parts of R (dR), by chunk parity
+  __device__ __forceinline__ f32x4 sum(int c, int v, int lane) const {
+    return (r[c & 1][v][0][lane] + r[c & 1][v][1][lane]) + (r[c & 1][v][2][lane] + r[c & 1][v][3][lane]);
+  }
+};
+// x[i] for a uniform i < 4
+__device__ __forceinline__ float pick4(const f32x4& x, int i) {
+  return i < 2 ? (i == 0 ? x[0] : x[1]) : (i == 2 ? x[2] : x[3]);
+}
 
-template <int D, int NWV, bool STASH, bool SCORE>
-__global__ void __launch_bounds__(64 * NWV) chan_scan_fwd_kernel(ChanArgs p) {
+// SCORE (|r_t| requested): each value tile's sum of squares of a token's net
+// write goes to the record's U, at the tile's first column, which only this
+// workgroup reads and has read; chan_rnorm_kernel sums them.
+template <int D, int NV, bool STASH, bool SCORE>
+__global__ void __launch_bounds__(256, 2) chan_split_fwd_kernel(ChanArgs p) {
   typedef ChRec<D> Rc;
-  typedef ChanScanFSmem<D, NWV> Sm;
-  constexpr int NT = 64 * NWV, NDT = D / 16, LDD = Sm::LDD, BV = Sm::BV, LDU = Sm::LDU, NVB = D / BV;
-  static_assert(!SCORE || NVB == 1, "the update norm sums over all value columns in one workgroup");
-  __shared__ Sm sm;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g4 = lane >> 4, n16 = lane & 15;
+  typedef ChSplit<D> Sp;
+  constexpr int KT = Sp::KT, PF = Sp::PF(NV, SCORE);
+  __shared__ ChanExchange<NV> sm, smy;   // parts of R, of Y
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g4 = lane >> 4, n16 = lane & 15;
   const int nchains = p.B * p.H;
-  const int work = xcd_remap(blockIdx.x, nchains * NVB);
-  const int chain = work / NVB, vb = work % NVB;
+  const int work = xcd_remap(blockIdx.x, nchains * (Sp::NVT / NV));   // a chain's workgroups read one record: one XCD
+  const int chain = work / (Sp::NVT / NV), V0 = NV * (work % (Sp::NVT / NV));
   const int h = chain % p.H, b = chain / p.H;
-  const int V = vb * NWV + wave;
   const int NC = (p.T + CC - 1) / CC;
   const size_t NR = (size_t)nchains * NC;
   const unsigned rsb = (unsigned)((size_t)p.H * D * 4);
 
-  f32x4 S[NDT];   // S[dt][i] = S0[16 dt + 4 g + i][16 V + n]
+  f32x4 S[NV][KT];   // S[v][t][i] = S0[16 (KT wave + t) + 4 g + i][16 (V0 + v) + n]
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) {
-    S[dt] = zero4();
-    if (p.s0) {
+  for (int v = 0; v < NV; ++v)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) S[dt][i] = p.s0[(size_t)chain * D * D + (dt * 16 + 4 * g4 + i) * D + 16 * V + n16];
+    for (int t = 0; t < KT; ++t) {
+      S[v][t] = zero4();
+      if (p.s0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          S[v][t][i] = p.s0[(size_t)chain * D * D + ((KT * wave + t) * 16 + 4 * g4 + i) * D + 16 * (V0 + v) + n16];
+      }
     }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-
-  Stage<float, CC, D, 1, NT> pn, pq;
-  Stage<float, D, CC, 1, NT> pk;
-  Stage<float, CC, CC, 1, NT> pa;
-  Stage<float, 1, D, 1, NT> pe;
-  Stage<float, CC, BV, 1, NT> pu;
-  auto fetch = [&](int c) {
-    const float* fr = p.frec + rec_index(chain, c, nchains) * Rc::FN;
-    pn.fetch_dense(fr + Rc::F_NWM, tid);
-    pq.fetch_dense(fr + Rc::F_QE, tid);
-    pk.fetch_dense(fr + Rc::F_KFT, tid);
-    pa.fetch_dense(fr + Rc::F_AQ, tid);
-    pe.fetch_dense(fr + Rc::F_EGL, tid);
-    pu.fetch(buf_rsrc(fr + Rc::F_U + vb * BV, (unsigned)(Rc::CD * 4)), (unsigned)(D * 4), tid);
+  struct Ops {
+    f32x4 nw[KT], qe[KT], kf[KT], eg[KT], u[NV];
+    float aq;   // column 4 g + wave of Aq: each wave takes a quarter of Aq R's sum
   };
-  fetch(0);
-  __builtin_amdgcn_s_waitcnt(0);
-
-  for (int c = 0; c < NC; ++c) {
-    const int t0 = c * CC;
+  const unsigned orow = (n16 * D + 4 * g4) * 4, ocol = (n16 * CC + 4 * g4) * 4, ou = (4 * g4 * D + n16) * 4, oe = 16 * g4;
+  auto fetch = [&](Ops& x, int c) {
+    load_fence();
+    const float* fr = p.frec + rec_index(chain, c, nchains) * Rc::FN;
+    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc((void*)fr, 0, Rc::FN * 4, 0x00020000);
+    const int kw = 16 * KT * wave;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      x.nw[t] = rec_load4(rr, orow, Rc::F_NWM + 16 * t + kw);
+      x.qe[t] = rec_load4(rr, orow, Rc::F_QE + 16 * t + kw);
+      x.kf[t] = rec_load4(rr, ocol, Rc::F_KFT + (16 * t + kw) * CC);
+      x.eg[t] = rec_load4(rr, oe, Rc::F_EGL + 16 * t + kw);
+    }
+    x.aq = rec_load1(rr, ocol, Rc::F_AQ + wave);
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x.u[v][s] = rec_load1(rr, ou, Rc::F_U + s * D + 16 * (V0 + v));
+    load_fence();
+  };
+  // chunk c's output from the waves' parts (one wave a tile, after the barrier that follows them)
+  auto y_out = [&](int c, int v) {
+    const f32x4 yt = tile_transpose((float*)nullptr, smy.sum(c, v, lane), lane);
+    const __amdgpu_buffer_rsrc_t yr = chunk_rsrc((const float*)p.y, b, c * CC, p.T, p.H, h, D);
+    buf_store4(yr, (unsigned)n16 * rsb + (16 * (V0 + v) + 4 * g4) * 4, (const float*)nullptr, yt[0], yt[1], yt[2], yt[3]);
+  };
+  auto step = [&](const Ops& x, int c) {
     const size_t rec = rec_index(chain, c, nchains);
-    __syncthreads();
-    pn.template commit_nat<LDD>(sm.nwm, tid);
-    pq.template commit_nat<LDD>(sm.qe, tid);
-    pk.template commit_nat<LDC>(sm.kft, tid);
-    pa.template commit_nat<LDC>(sm.aq, tid);
-    pe.template commit_nat<D>(sm.egl, tid);
-    pu.template commit_nat<LDU>(sm.u, tid);
-    __syncthreads();
-    fetch(min(c + 1, NC - 1));
     if constexpr (STASH) {
       float* cst = (float*)p.chunk_states + rec * (D * D);
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) *(f32x4*)(cst + stash_tile_offset<float, D>(dt, V, lane)) = S[dt];
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+          *(f32x4*)(cst + stash_tile_offset<float, D>(KT * wave + t, V0 + v, lane)) = S[v][t];
     }
-    // R = U - Wm S0 (two accumulators)
-    f32x4 R0, R1 = zero4();
+    // this wave's keys of R = U - Wm S0 (U with wave 0) and of (Q o e^G) S0
 #pragma unroll
-    for (int s = 0; s < 4; ++s) R0[s] = sm.u[(4 * g4 + s) * LDU + 16 * wave + n16];
-#pragma unroll
-    for (int kb = 0; kb < NDT; ++kb) mma((kb & 1) ? R1 : R0, ld_frag(&sm.nwm[n16 * LDD + kb * 16], g4), S[kb]);
-    const f32x4 R = R0 + R1;
-    if constexpr (STASH) {
-      float* rst = (float*)p.chunk_states + NR * D * D + rec * (CC * D);
-      *(f32x4*)(rst + stash_tile_offset<float, D>(0, V, lane)) = R;
+    for (int v = 0; v < NV; ++v) {
+      f32x4 r = wave == 0 ? x.u[v] : zero4(), r1 = zero4();
+      mma2(r, r1, x.nw, S[v]);
+      sm.r[c & 1][v][wave][lane] = r + r1;
     }
-    if constexpr (SCORE) {
-      const f32x4 sq = R * R;
+    lds_barrier();
+    f32x4 y[NV], R[NV];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float x = row_prefix16(sq[e]);
-        if (n16 == 15) sm.rn[wave][4 * g4 + e] = x;
-      }
-    }
-    // Y = (Q o e^G) S0 + Aq R
-    {
-      f32x4 Y0 = zero4(), Y1 = zero4();
-#pragma unroll
-      for (int kb = 0; kb < NDT; ++kb) mma((kb & 1) ? Y1 : Y0, ld_frag(&sm.qe[n16 * LDD + kb * 16], g4), S[kb]);
-      mma(Y0, ld_frag(&sm.aq[n16 * LDC], g4), R);
-      const f32x4 yt = tile_transpose((float*)nullptr, Y0 + Y1, lane);
-      const __amdgpu_buffer_rsrc_t yr = chunk_rsrc((const float*)p.y, b, t0, p.T, p.H, h, D);
-      buf_store4(yr, (unsigned)n16 * rsb + (16 * V + 4 * g4) * 4, (const float*)nullptr, yt[0], yt[1], yt[2], yt[3]);
+    for (int v = 0; v < NV; ++v) {   // (while the parts arrive)
+      f32x4 y1 = zero4();
+      y[v] = zero4();
+      mma2(y[v], y1, x.qe, S[v]);
+      y[v] += y1;
     }
     // S = diag(e^{G_L}) S0 + (K o e^{G_L - G})^T R
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      S[dt] *= *(const f32x4*)&sm.egl[dt * 16 + 4 * g4];
-      mma(S[dt], ld_frag(&sm.kft[(dt * 16 + n16) * LDC], g4), R);
-    }
-    if constexpr (SCORE) {
-      __syncthreads();
-      if (tid < CC && t0 + tid < p.T) {
-        float s = 0.f;
+    for (int v = 0; v < NV; ++v) {
+      R[v] = sm.sum(c, v, lane);
 #pragma unroll
-        for (int w = 0; w < NWV; ++w) s += sm.rn[w][tid];
-        p.r_norm[((size_t)b * p.T + t0 + tid) * p.H + h] = sqrtf(s);
+      for (int t = 0; t < KT; ++t) {
+        S[v][t] *= x.eg[t];
+        mma(S[v][t], x.kf[t], R[v]);
       }
     }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      smy.r[c & 1][v][wave][lane] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.aq, pick4(R[v], wave), y[v], 0, 0, 0);
+      if (c > 0 && wave == ((c + 1 + v) & 3)) y_out(c - 1, v);
+      if constexpr (STASH)
+        if (wave == ((c + 2 + v) & 3)) {
+          float* rst = (float*)p.chunk_states + NR * D * D + rec * (CC * D);
+          *(f32x4*)(rst + stash_tile_offset<float, D>(0, V0 + v, lane)) = R[v];
+        }
+      if constexpr (SCORE)
+        if (wave == 0) {   // (U's reader)
+          float* fr = p.frec + rec * Rc::FN;
+          const f32x4 sq = R[v] * R[v];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float n2 = row_prefix16(sq[e]);
+            if (n16 == 15) fr[Rc::F_U + (4 * g4 + e) * D + 16 * (V0 + v)] = n2;
+          }
+        }
+    }
+  };
+  Ops x[PF];
+#pragma unroll
+  for (int j = 0; j < PF; ++j) {
+    fetch(x[j], min(j, NC - 1));   // (in order: a chunk's wait leaves the later ones in flight)
   }
-  if (p.s_out) {
+#pragma clang loop unroll(disable)
+  for (int c0 = 0; c0 < NC; c0 += PF) {   // (one exit, and the same loads in flight on every path)
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+    for (int j = 0; j < PF; ++j) {
+      if (c0 + j < NC) step(x[j], c0 + j);
+      fetch(x[j], min(c0 + j + PF, NC - 1));
+    }
+  }
+  lds_barrier();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p.s_out[(size_t)chain * D * D + (dt * 16 + 4 * g4 + i) * D + 16 * V + n16] = S[dt][i];
+  for (int v = 0; v < NV; ++v) {
+    if (NC > 0 && wave == (v & 3)) y_out(NC - 1, v);
+    if (p.s_out) {
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          p.s_out[(size_t)chain * D * D + ((KT * wave + t) * 16 + 4 * g4 + i) * D + 16 * (V0 + v) + n16] = S[v][t][i];
+    }
   }
 }
 
-// ---------------------------------------------------------------------------
-// reverse scan of the state gradient, value-split like the forward:
+template <int D>
+__global__ void __launch_bounds__(256) chan_rnorm_kernel(ChanArgs p) {
+  typedef ChRec<D> Rc;
+  const int nchains = p.B * p.H;
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;   // (chain, token)
+  if (i >= (long long)nchains * p.T) return;
+  const int t = (int)(i % p.T), chain = (int)(i / p.T), h = chain % p.H, b = chain / p.H;
+  const float* u = p.frec + rec_index(chain, t / CC, nchains) * Rc::FN + Rc::F_U + (t % CC) * D;
+  float s = 0.f;
+#pragma unroll
+  for (int V = 0; V < D / 16; ++V) s += u[16 * V];
+  p.r_norm[((size_t)b * p.T + t) * p.H + h] = sqrtf(s);
+}
+
+// reverse scan of the state gradient:
 //   dR = Aq^T dY + (K o e^{G_L - G}) dS,  dB = T^T dR
 //   dS0 = diag(e^{G_L}) dS + (Q o e^G)^T dY - (K o e^G)^T diag(beta_e) dB
-// ---------------------------------------------------------------------------
-template <int D, int NWV>
-struct alignas(16) ChanScanBSmem {
-  static constexpr int LDD = D + 4, BV = 16 * NWV;
-  float kf[CC * LDD];
-  float qet[D * LDC];
-  float ket[D * LDC];
-  float tt[CC * LDC];
-  float aqt[CC * LDC];
-  float be[CC];
-  float egl[D];
-  float dyt[BV * LDC];
-};
-
-template <int D, int NWV>
-__global__ void __launch_bounds__(64 * NWV) chan_scan_bwd_kernel(ChanBwdArgs p) {
+// where (K o e^G)^T diag(beta_e) T^T = Wm^T, so dS takes dR itself and dB is
+// only formed for the stash
+template <int D, int NV>
+__global__ void __launch_bounds__(256, 2) chan_split_bwd_kernel(ChanBwdArgs p) {
   typedef ChRec<D> Rc;
-  typedef ChanScanBSmem<D, NWV> Sm;
-  constexpr int NT = 64 * NWV, NDT = D / 16, LDD = Sm::LDD, BV = Sm::BV, NVB = D / BV;
-  __shared__ Sm sm;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g4 = lane >> 4, n16 = lane & 15;
+  typedef ChSplit<D> Sp;
+  constexpr int KT = Sp::KT, PF = Sp::PF(NV, false);
+  __shared__ ChanExchange<NV> sm;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g4 = lane >> 4, n16 = lane & 15;
   const int nchains = p.B * p.H;
-  const int work = xcd_remap(blockIdx.x, nchains * NVB);
-  const int chain = work / NVB, vb = work % NVB;
+  const int work = xcd_remap(blockIdx.x, nchains * (Sp::NVT / NV));
+  const int chain = work / (Sp::NVT / NV), V0 = NV * (work % (Sp::NVT / NV));
   const int h = chain % p.H, b = chain / p.H;
-  const int V = vb * NWV + wave;
   const int NC = (p.T + CC - 1) / CC;
   const size_t NR = (size_t)nchains * NC;
   const float* brec = (const float*)p.s_stash + NR * ((size_t)D * D + CC * D + Rc::FN);
 
-  f32x4 dS[NDT];
+  f32x4 dS[NV][KT];
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) {
-    dS[dt] = zero4();
-    if (p.ds_final) {
+  for (int v = 0; v < NV; ++v)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        dS[dt][i] = p.ds_final[(size_t)chain * D * D + (dt * 16 + 4 * g4 + i) * D + 16 * V + n16];
+    for (int t = 0; t < KT; ++t) {
+      dS[v][t] = zero4();
+      if (p.ds_final) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          dS[v][t][i] = p.ds_final[(size_t)chain * D * D + ((KT * wave + t) * 16 + 4 * g4 + i) * D + 16 * (V0 + v) + n16];
+      }
     }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-
-  Stage<float, CC, D, 1, NT> pf;
-  Stage<float, D, CC, 1, NT> pqt, pkt;
-  Stage<float, CC, CC, 1, NT> ptt, pat;
-  Stage<float, 1, CC, 1, NT> pb;
-  Stage<float, 1, D, 1, NT> pe;
-  Stage<float, CC, BV, 4, NT> py;
-  const unsigned rsb = (unsigned)((size_t)p.H * D * 4);
-  auto fetch = [&](int c) {
-    const float* br = brec + rec_index(chain, c, nchains) * Rc::BN;
-    pf.fetch_dense(br + Rc::B_KF, tid);
-    pqt.fetch_dense(br + Rc::B_QET, tid);
-    pkt.fetch_dense(br + Rc::B_KET, tid);
-    ptt.fetch_dense(br + Rc::B_TT, tid);
-    pat.fetch_dense(br + Rc::B_AQT, tid);
-    pb.fetch_dense(br + Rc::B_BE, tid);
-    pe.fetch_dense(br + Rc::B_EGL, tid);
-    py.fetch(chunk_rsrc(p.dy + vb * BV, b, c * CC, p.T, p.H, h, D), rsb, tid);
+  struct Ops {
+    f32x4 kf[KT], qt[KT], nw[KT], eg[KT], tt, dy[NV];
+    float at;   // column 4 g + wave of Aq^T: each wave takes a quarter of Aq^T dY's sum
   };
-  fetch(NC - 1);
-  __builtin_amdgcn_s_waitcnt(0);
-
-  for (int c = NC - 1; c >= 0; --c) {
+  const unsigned orow = (n16 * D + 4 * g4) * 4, ocol = (n16 * CC + 4 * g4) * 4, oe = 16 * g4;
+  auto fetch = [&](Ops& x, int c) {
+    load_fence();
+    const float* br = brec + rec_index(chain, c, nchains) * Rc::BN;
+    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc((void*)br, 0, Rc::BN * 4, 0x00020000);
+    const int kw = 16 * KT * wave;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      x.kf[t] = rec_load4(rr, orow, Rc::B_KF + 16 * t + kw);
+      x.qt[t] = rec_load4(rr, ocol, Rc::B_QET + (16 * t + kw) * CC);
+      x.nw[t] = rec_load4(rr, ocol, Rc::B_NWT + (16 * t + kw) * CC);
+      x.eg[t] = rec_load4(rr, oe, Rc::B_EGL + 16 * t + kw);
+    }
+    x.tt = rec_load4(rr, ocol, Rc::B_TT);
+    x.at = rec_load1(rr, ocol, Rc::B_AQT + wave);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {   // dY as a B operand; rows past T (masked where used) read the last
+      const int t = min(c * CC + 4 * g4 + s, p.T - 1);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) x.dy[v][s] = p.dy[(((size_t)b * p.T + t) * p.H + h) * D + 16 * (V0 + v) + n16];
+    }
+    load_fence();
+  };
+  auto step = [&](const Ops& x, int c) {
     const size_t rec = rec_index(chain, c, nchains);
-    __syncthreads();
-    pf.template commit_nat<LDD>(sm.kf, tid);
-    pqt.template commit_nat<LDC>(sm.qet, tid);
-    pkt.template commit_nat<LDC>(sm.ket, tid);
-    ptt.template commit_nat<LDC>(sm.tt, tid);
-    pat.template commit_nat<LDC>(sm.aqt, tid);
-    pb.template commit_nat<CC>(sm.be, tid);
-    pe.template commit_nat<D>(sm.egl, tid);
-    py.template commit_tr<LDC>(sm.dyt, tid);
-    __syncthreads();
-    fetch(max(c - 1, 0));
-    {
-      float* cst = (float*)p.ds_stash + rec * (D * D);
+    float* cst = (float*)p.ds_stash + rec * (D * D);
+    f32x4 dY[NV];
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) *(f32x4*)(cst + stash_tile_offset<float, D>(dt, V, lane)) = dS[dt];
+    for (int v = 0; v < NV; ++v) {
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+        *(f32x4*)(cst + stash_tile_offset<float, D>(KT * wave + t, V0 + v, lane)) = dS[v][t];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) dY[v][s] = c * CC + 4 * g4 + s < p.T ? x.dy[v][s] : 0.f;
+      f32x4 r = zero4(), r1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.at, pick4(dY[v], wave), zero4(), 0, 0, 0);
+      mma2(r, r1, x.kf, dS[v]);
+      sm.r[c & 1][v][wave][lane] = r + r1;
     }
-    const f32x4 dYf = ld_frag(&sm.dyt[(16 * wave + n16) * LDC], g4);
-    f32x4 dR0 = zero4(), dR1 = zero4();
+    lds_barrier();
 #pragma unroll
-    for (int kb = 0; kb < NDT; ++kb) mma((kb & 1) ? dR1 : dR0, ld_frag(&sm.kf[n16 * LDD + kb * 16], g4), dS[kb]);
-    mma(dR0, ld_frag(&sm.aqt[n16 * LDC], g4), dYf);
-    const f32x4 dR = dR0 + dR1;
-    f32x4 dB = zero4();
-    mma(dB, ld_frag(&sm.tt[n16 * LDC], g4), dR);
-    {
-      float* bst = (float*)p.ds_stash + NR * D * D + rec * (CC * D);
-      *(f32x4*)(bst + stash_tile_offset<float, D>(0, V, lane)) = dB;
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {   // (while the parts arrive)
+        dS[v][t] *= x.eg[t];
+        mma(dS[v][t], x.qt[t], dY[v]);
+      }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const f32x4 dR = sm.sum(c, v, lane);
+#pragma unroll
+      for (int t = 0; t < KT; ++t) mma(dS[v][t], x.nw[t], dR);
+      if (wave == ((c + v) & 3)) {
+        f32x4 dB = zero4();
+        mma(dB, x.tt, dR);
+        float* bst = (float*)p.ds_stash + NR * D * D + rec * (CC * D);
+        *(f32x4*)(bst + stash_tile_offset<float, D>(0, V0 + v, lane)) = dB;
+      }
     }
-    const f32x4 dBf = -dB * *(const f32x4*)&sm.be[4 * g4];
+  };
+  Ops x[PF];
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      dS[dt] *= *(const f32x4*)&sm.egl[dt * 16 + 4 * g4];
-      mma(dS[dt], ld_frag(&sm.qet[(dt * 16 + n16) * LDC], g4), dYf);
-      mma(dS[dt], ld_frag(&sm.ket[(dt * 16 + n16) * LDC], g4), dBf);
+  for (int j = 0; j < PF; ++j) {
+    fetch(x[j], max(NC - 1 - j, 0));
+  }
+#pragma clang loop unroll(disable)
+  for (int c0 = NC - 1; c0 >= 0; c0 -= PF) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      if (c0 - j >= 0) step(x[j], c0 - j);
+      fetch(x[j], max(c0 - j - PF, 0));
     }
   }
   if (p.ds0) {
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+    for (int v = 0; v < NV; ++v)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p.ds0[(size_t)chain * D * D + (dt * 16 + 4 * g4 + i) * D + 16 * V + n16] = dS[dt][i];
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          p.ds0[(size_t)chain * D * D + ((KT * wave + t) * 16 + 4 * g4 + i) * D + 16 * (V0 + v) + n16] = dS[v][t][i];
   }
 }
 
@@ -721,6 +817,29 @@ __global__ void __launch_bounds__(64 * (D / 16)) chan_grads_kernel(ChanBwdArgs p
   }
 }
 
+// Value tiles per workgroup of the scans: one while each of the 256 CUs
+// gets one workgroup at most (the step's latency counts), two up to two full
+// rounds of the chip, four beyond (a record is read D / 64 times instead of D / 16, and
+// more products stand between two barriers).  Times with the prep and, in
+// training, the gradient kernel, T = 512 training (1 | 2 | 4 tiles) at d = 128:
+// 64 chains 512 | 488 | 548 us, 96: 750 | 728 | 717, 128: 971 | 887 | 864, 256:
+// 1829 | 1670 | 1574; T = 1024 without gradient, 64 chains 328 | 320 | 389.
+static int chan_tiles(int nchains, int D) {
+  const long long tiles = (long long)nchains * (D / 16);
+  return tiles <= 256 ? 1 : tiles < 1024 ? 2 : 4;
+}
+
+template <int D, int NV>
+static int launch_chan_scan(const ChanArgs& a, hipStream_t stream) {
+  const dim3 grid(a.B * a.H * (ChSplit<D>::NVT / NV)), block(256);
+  const bool train = a.chunk_states != nullptr;
+  if (train && a.r_norm) hipLaunchKernelGGL((chan_split_fwd_kernel<D, NV, true, true>), grid, block, 0, stream, a);
+  else if (train) hipLaunchKernelGGL((chan_split_fwd_kernel<D, NV, true, false>), grid, block, 0, stream, a);
+  else if (a.r_norm) hipLaunchKernelGGL((chan_split_fwd_kernel<D, NV, false, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((chan_split_fwd_kernel<D, NV, false, false>), grid, block, 0, stream, a);
+  return check_launch("chan_split_fwd_kernel");
+}
+
 template <int D>
 static int launch_chan_fwd(ChanArgs a, hipStream_t stream) {
   typedef ChRec<D> Rc;
@@ -735,28 +854,24 @@ static int launch_chan_fwd(ChanArgs a, hipStream_t stream) {
     hipLaunchKernelGGL((chan_prep_kernel<D, false>), dim3(nchains * NC), dim3(64 * (D / 16)), 0, stream, a);
   int rc = check_launch("chan_prep_kernel");
   if (rc) return rc;
-  if (a.r_norm) {   // one workgroup per chain: the update norm sums every value column
-    constexpr int NW = D / 16;
-    if (train)
-      hipLaunchKernelGGL((chan_scan_fwd_kernel<D, NW, true, true>), dim3(nchains), dim3(64 * NW), 0, stream, a);
-    else
-      hipLaunchKernelGGL((chan_scan_fwd_kernel<D, NW, false, true>), dim3(nchains), dim3(64 * NW), 0, stream, a);
-  } else {
-    constexpr int NW = 4, NVB = D / 64;
-    if (train)
-      hipLaunchKernelGGL((chan_scan_fwd_kernel<D, NW, true, false>), dim3(nchains * NVB), dim3(64 * NW), 0, stream, a);
-    else
-      hipLaunchKernelGGL((chan_scan_fwd_kernel<D, NW, false, false>), dim3(nchains * NVB), dim3(64 * NW), 0, stream, a);
-  }
-  return check_launch("chan_scan_fwd_kernel");
+  const int nv = chan_tiles(nchains, D);
+  rc = nv == 1 ? launch_chan_scan<D, 1>(a, stream)
+               : nv == 2 ? launch_chan_scan<D, 2>(a, stream) : launch_chan_scan<D, 4>(a, stream);
+  if (rc || !a.r_norm) return rc;
+  const long long n = (long long)nchains * a.T;
+  hipLaunchKernelGGL((chan_rnorm_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a);
+  return check_launch("chan_rnorm_kernel");
 }
 
 template <int D>
 static int launch_chan_bwd(const ChanBwdArgs& a, hipStream_t stream) {
   const int NC = (a.T + CC - 1) / CC;
-  constexpr int NW = 4, NVB = D / 64;
-  hipLaunchKernelGGL((chan_scan_bwd_kernel<D, NW>), dim3(a.B * a.H * NVB), dim3(64 * NW), 0, stream, a);
-  int rc = check_launch("chan_scan_bwd_kernel");
+  const int nv = chan_tiles(a.B * a.H, D);
+  const dim3 grid(a.B * a.H * (ChSplit<D>::NVT / nv)), block(256);
+  if (nv == 1) hipLaunchKernelGGL((chan_split_bwd_kernel<D, 1>), grid, block, 0, stream, a);
+  else if (nv == 2) hipLaunchKernelGGL((chan_split_bwd_kernel<D, 2>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((chan_split_bwd_kernel<D, 4>), grid, block, 0, stream, a);
+  int rc = check_launch("chan_split_bwd_kernel");
   if (rc) return rc;
   hipLaunchKernelGGL((chan_grads_kernel<D>), dim3(a.B * a.H * NC), dim3(64 * (D / 16)), 0, stream, a);
   return check_launch("chan_grads_kernel");

@@ -161,8 +161,10 @@ struct alignas(16) ChanPrepSmem {
   float vt[D * LDC];     // V^T
 };
 
+// (registers held to two workgroups a CU at d = 128, 130 -> 128: prep 64 -> 45 us
+// at B = 1, T = 2048, H = 16, 36 -> 29 us with the backward's records at 32 chains)
 template <int D, bool BWD>
-__global__ void __launch_bounds__(64 * (D / 16)) chan_prep_kernel(ChanArgs p) {
+__global__ void __launch_bounds__(64 * (D / 16), D == 128 ? 4 : 3) chan_prep_kernel(ChanArgs p) {
   typedef ChD<D> Cd;
   typedef ChRec<D> Rc;
   constexpr int NT = Cd::NT, LDD = Cd::LDD;
@@ -619,8 +621,12 @@ struct alignas(16) ChanGradSmem {
   float red[2][ChD<D>::NW][CC];   // per-wave partial row sums: dbeta_e, dbeta_w
 };
 
+// Bound by the latency of its LDS reads and by how many workgroups hide it:
+// registers are held to what lets LDS's two (d = 128; three at 64) stay on a CU
+// (128 of them; at 138, and with a branch and single LDS reads per pair of
+// tokens, one did).  B = 2, T = 512, H = 16, d = 128: 108 -> 80 us.
 template <int D>
-__global__ void __launch_bounds__(64 * (D / 16)) chan_grads_kernel(ChanBwdArgs p) {
+__global__ void __launch_bounds__(64 * (D / 16), D == 128 ? 4 : 3) chan_grads_kernel(ChanBwdArgs p) {
   typedef ChD<D> Cd;
   constexpr int NW = Cd::NW, NT = Cd::NT, NDT = Cd::NDT, LDD = Cd::LDD;
   __shared__ ChanGradSmem<D> sm;
@@ -714,41 +720,53 @@ __global__ void __launch_bounds__(64 * (D / 16)) chan_grads_kernel(ChanBwdArgs p
     mma(P2, ld_frag(&sm.dB[n16 * LDD + kb * 16], g4), Sf);
     mma(P3, ld_frag(&sm.R[n16 * LDD + kb * 16], g4), dSf);
   }
-  // lane (g, n): rows i = 4 g + ii of column d; the column's operands in registers
-  float Gc[CC], kc[CC], qc[CC];
-#pragma unroll
-  for (int j = 0; j < CC; ++j) {
-    Gc[j] = o.G[j * LDD + d];
-    kc[j] = o.k[j * LDD + d];
-    qc[j] = o.q[j * LDD + d];
-  }
-  const float GL = Gc[CC - 1];
-  float dq[4], dk[4], dG[4], dGLp = 0.f, pbe[4];
+  // lane (g, n): rows i = 4 g + ii of column d
+  const float GL = o.G[(CC - 1) * LDD + d];
+  float dq[4], dk[4], dG[4], dGLp = 0.f, pbe[4], Gi[4], ki[4], qi[4], bei[4];
 #pragma unroll
   for (int ii = 0; ii < 4; ++ii) {
     const int i = 4 * g4 + ii;
-    const float E = __expf(Gc[i]), F = __expf(GL - Gc[i]);
-    const float bei = o.be[i];
+    Gi[ii] = o.G[i * LDD + d];
+    ki[ii] = o.k[i * LDD + d];
+    qi[ii] = o.q[i * LDD + d];
+    bei[ii] = o.be[i];
+    const float E = __expf(Gi[ii]), F = __expf(GL - Gi[ii]);
     dq[ii] = E * P1[ii];
-    dk[ii] = -bei * E * P2[ii] + F * P3[ii];
-    dG[ii] = E * (qc[i] * P1[ii] - bei * kc[i] * P2[ii]) - F * kc[i] * P3[ii];
-    dGLp += F * kc[i] * P3[ii];
-    pbe[ii] = -E * kc[i] * P2[ii];
-    // grams, row i as the query / erase side (j <= i) and as the key side (i <= j')
+    dk[ii] = -bei[ii] * E * P2[ii] + F * P3[ii];
+    dG[ii] = E * (qi[ii] * P1[ii] - bei[ii] * ki[ii] * P2[ii]) - F * ki[ii] * P3[ii];
+    dGLp += F * ki[ii] * P3[ii];
+    pbe[ii] = -E * ki[ii] * P2[ii];
+  }
+  // grams, row i as the query / erase side (j <= i) and as the key side
+  // (i <= j).  The prefix never rises, so that one exponential of -|G_i - G_j|
+  // serves both; what a row does not take is selected away (a NaN of a later
+  // token stays there), so that no lane branches and the LDS reads, four
+  // values each, run ahead of the sums.
+#pragma unroll 1   // (all blocks' reads at once would spill)
+  for (int jb = 0; jb < CC / 4; ++jb) {
+    f32x4 ar[4], lr[4];
 #pragma unroll
-    for (int j = 0; j < CC; ++j) {
-      if (j <= i) {
-        const float ex = __expf(Gc[i] - Gc[j]);
-        const float t1 = sm.dAq[i * LDC + j] * ex, t2 = sm.dL[i * LDC + j] * bei * ex;
-        dq[ii] += t1 * kc[j];
-        dk[ii] += t2 * kc[j];
-        dG[ii] += (t1 * qc[i] + t2 * kc[i]) * kc[j];
-      }
-      if (j >= i) {
-        const float ex = __expf(Gc[j] - Gc[i]);
-        const float cc = (sm.dAq[j * LDC + i] * qc[j] + sm.dL[j * LDC + i] * o.be[j] * kc[j]) * ex;
-        dk[ii] += cc;
-        dG[ii] -= cc * kc[i];
+    for (int ii = 0; ii < 4; ++ii) {
+      ar[ii] = *(const f32x4*)&sm.dAq[(4 * g4 + ii) * LDC + 4 * jb];
+      lr[ii] = *(const f32x4*)&sm.dL[(4 * g4 + ii) * LDC + 4 * jb];
+    }
+    const f32x4 bej = *(const f32x4*)&o.be[4 * jb];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int j = 4 * jb + jj;
+      const float Gj = o.G[j * LDD + d], kj = o.k[j * LDD + d], qj = o.q[j * LDD + d];
+      const f32x4 ac = *(const f32x4*)&sm.dAq[j * LDC + 4 * g4], lc = *(const f32x4*)&sm.dL[j * LDC + 4 * g4];
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) {
+        const bool lo = j <= 4 * g4 + ii, hi = j >= 4 * g4 + ii;
+        const float ex = __expf(-fabsf(Gi[ii] - Gj));
+        const float t1 = ar[ii][jj] * ex, t2 = lr[ii][jj] * bei[ii] * ex;
+        const float cc = (ac[ii] * qj + lc[ii] * bej[jj] * kj) * ex;
+        dq[ii] += lo ? t1 * kj : 0.f;
+        dk[ii] += lo ? t2 * kj : 0.f;
+        dG[ii] += lo ? (t1 * qi[ii] + t2 * ki[ii]) * kj : 0.f;
+        dk[ii] += hi ? cc : 0.f;
+        dG[ii] -= hi ? cc * ki[ii] : 0.f;
       }
     }
   }
@@ -820,8 +838,9 @@ __global__ void __launch_bounds__(64 * (D / 16)) chan_grads_kernel(ChanBwdArgs p
 // Value tiles per workgroup of the scans: one while each of the 256 CUs
 // gets one workgroup at most (the step's latency counts), two up to two full
 // rounds of the chip, four beyond (a record is read D / 64 times instead of D / 16, and
-// more products stand between two barriers).  Times with the prep and, in
-// training, the gradient kernel, T = 512 training (1 | 2 | 4 tiles) at d = 128:
+// more products stand between two barriers).  Times of the
+// whole call, the gradient kernel at 108 us per 32 chains then, T = 512 training
+// (1 | 2 | 4 tiles) at d = 128:
 // 64 chains 512 | 488 | 548 us, 96: 750 | 728 | 717, 128: 971 | 887 | 864, 256:
 // 1829 | 1670 | 1574; T = 1024 without gradient, 64 chains 328 | 320 | 389.
 static int chan_tiles(int nchains, int D) {

@@ -38,7 +38,9 @@ template <> struct FragT<float> {
 __device__ __forceinline__ void mma(f32x4& acc, const bf16x8& a, const bf16x8& b) {
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
 }
-__device__ __forceinline__ void mma(f32x4& acc, const f32x4& a, const f32x4& b) {
+// (operands by value: acc may be one of them, and is written after every
+// quarter of the product)
+__device__ __forceinline__ void mma(f32x4& acc, const f32x4 a, const f32x4 b) {
   acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], b[0], acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], b[1], acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], b[2], acc, 0, 0, 0);

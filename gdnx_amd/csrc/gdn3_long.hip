@@ -23,15 +23,18 @@
 // rows of the Kronecker matrix in registers, which leaves one dependent 16 x
 // 16 x 16 product per sub-chunk; H and Q reach it through LDS as fragments.
 //
-// Bound: issue and latency of two waves per SIMD (about 1,300 vector and 170
-// matrix instructions per wave and batch; the token rows of the next batch are
-// loaded under the second half of this one).  B = 1, T = 32768, H = 16, 4 lanes,
-// d = 128, bf16, a compaction every 2048 tokens (64 chains, 8 runs): 60 us a
-// second pass and 39 us a first pass per interval against 305 us for the
-// walk of the sub-chunks one by one on 8 workgroups per chain that this
-// replaced; the call 5.27 -> 2.0 ms.  256, 512 and 1024 chains over 512-token
-// intervals: 0.98 -> 0.46, 0.93 -> 0.34, 1.06 -> 0.45 ms.  A single batch per
-// interval (a compaction every 64 tokens, 64 chains): 1.37 -> 1.25 ms.
+// The 16 x 16 x 16 algebra (the inverse, W, T X, W U, Qo U, Aq U) and the decays
+// are float32 whatever the IO type: where a sub-chunk's keys are alike (repeated
+// tokens) the inverse's factors reach (1 + l)^15, l its largest entry, and cancel.
+// As hi + lo bf16 parts (2^-17) those products left 5.5e-4 in U for unit keys of one
+// direction and 2.4e-2 for |k| = 2; in float32 8e-6 and 5e-4 (the call below
+// took 2.00 ms with the parts).
+//
+// Bound: issue and latency of two waves per SIMD (the token rows of the next
+// batch are loaded under the second half of this one).  B = 1, T = 32768, H =
+// 16, 4 lanes, d = 128, bf16, a compaction every 2048 tokens (64 chains, 8
+// runs), against the walk of the sub-chunks one by one on 8 workgroups per chain
+// that this replaced: the call 5.24 -> 2.14 ms.
 #include <utility>
 
 #include "gdn3_common.hpp"
@@ -39,49 +42,6 @@
 
 namespace gdnx {
 namespace {
-
-// Operands of a 16 x 16 x 16 product of fp32 values, four k a lane (k = 4 g + e).
-// float32 IO: fp32 MFMA (four instructions of 32 cycles).  bf16 IO: each
-// value as hi + lo bf16 parts, the two halves of a 32-wide bf16 k-step, so two
-// instructions of 16 cycles form all four cross products; an operand is within
-// 2^-17 of its fp32 value, far inside what bf16 h, q, k and v leave (U stays
-// 2e-4, y 1.7e-3 from the same in 64 bits either way).
-template <typename CT> struct Op16;
-template <> struct Op16<float> {
-  typedef f32x4 A;
-  typedef f32x4 B;
-  static __device__ __forceinline__ A a(const f32x4& x) { return x; }
-  static __device__ __forceinline__ B b(const f32x4& x) { return x; }
-};
-template <> struct Op16<bf16> {
-  typedef bf16x8 A;                  // [hi | lo]
-  struct B { bf16x8 h, l; };         // [hi | hi], [lo | lo]
-  static __device__ __forceinline__ void split(const f32x4& x, bf16x4& h, bf16x4& l) {
-    h = __builtin_convertvector(x, bf16x4);
-    l = __builtin_convertvector(x - __builtin_convertvector(h, f32x4), bf16x4);
-  }
-  static __device__ __forceinline__ A a(const f32x4& x) {
-    bf16x4 h, l;
-    split(x, h, l);
-    return __builtin_shufflevector(h, l, 0, 1, 2, 3, 4, 5, 6, 7);
-  }
-  static __device__ __forceinline__ B b(const f32x4& x) {
-    bf16x4 h, l;
-    split(x, h, l);
-    return B{__builtin_shufflevector(h, h, 0, 1, 2, 3, 0, 1, 2, 3), __builtin_shufflevector(l, l, 0, 1, 2, 3, 0, 1, 2, 3)};
-  }
-};
-__device__ __forceinline__ void mma16(f32x4& acc, const f32x4& a, const f32x4& b) { mma(acc, a, b); }
-__device__ __forceinline__ void mma16(f32x4& acc, const bf16x8& a, const Op16<bf16>::B& b) {
-  mma(acc, a, b.h);
-  mma(acc, a, b.l);
-}
-// decays: the hardware exponential is within 1e-6 of e^x over the range
-// that matters, far inside bf16 operands
-template <typename CT> __device__ __forceinline__ float decay_exp(float x) {
-  if constexpr (sizeof(CT) == 2) return __expf(x);
-  else return expf(x);
-}
 
 constexpr int kBatch = 4;   // sub-chunks a workgroup prepares at once, one per wave
 
@@ -91,7 +51,7 @@ struct G3RunSmem {
   typedef typename FragT<CT>::type Frag;
   Frag hx[kBatch][KB][64];                                  // H rows of the batch as A fragments
   Frag qx[kBatch][KB][64];                                  // Q rows
-  typename Op16<CT>::A mt[kBatch][2 + 2 * NB][64];          // T, Aq, -W_b, Qo_b as A operands
+  f32x4 mt[kBatch][2 + 2 * NB][64];                         // T, Aq, -W_b, Qo_b as A operands
   alignas(16) CT vx[kBatch][kSC][D + 8];                    // V rows
   alignas(16) float aw[kBatch][kSC];                        // alpha w (per-channel gates: alpha)
   alignas(16) float kco[kBatch][kSC], qco[kBatch][kSC];     // alpha e^{2 (Gacc + G)}, e^{2 (Gacc + G)}
@@ -105,7 +65,6 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   typedef G3RunSmem<CT, D, P> Sm;
   typedef typename FragT<CT>::type Frag;
   typedef G3D<D> Ge;
-  typedef Op16<CT> Op;
   constexpr int NB = Sm::NB, KS = FragT<CT>::KSTEP, KB = Sm::KB, EPL = KS / 4;   // elements a lane holds of a k-step
   constexpr int TPW = D / 64;                                                     // value tiles per wave
   static_assert(sizeof(Frag) == 16 && EPL * sizeof(CT) == 16, "a fragment is one 16-byte load");
@@ -243,12 +202,6 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   }
 
-  typename Op::B ub[NB][TU];   // uo as operands
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int a = 0; a < TU; ++a) ub[b][a] = Op::b(uo[b][a]);
-
   if (FULL && ce == p.c1 && wave == 3) {   // suf[x]: the log decay after token 16 c1 - 128 + x
     const float a = lane_prefix<64>(lgtok(kSC * p.c1 - 128 + lane), lane);
     const float b = lane_prefix<64>(lgtok(kSC * p.c1 - 64 + lane), lane);
@@ -331,31 +284,30 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int i = 4 * g4 + e;
         gi[e] = __shfl(gl, i, 64);
         ai[e] = __shfl(alpha_l, i, 64);
-        xa[e] = n16 < i ? ai[e] * decay_exp<CT>(gi[e] - gl) * xa[e] : 0.f;
-        const float dn = n16 >= i ? decay_exp<CT>(gl - gi[e]) : 0.f;   // (row j = i here, column the later token)
+        xa[e] = n16 < i ? ai[e] * expf(gi[e] - gl) * xa[e] : 0.f;
+        const float dn = n16 >= i ? expf(gl - gi[e]) : 0.f;   // (row j = i here, column the later token)
         xt[e] = n16 > i ? alpha_l * dn * xt[e] : 0.f;
         if constexpr (FULL) aq[e] *= dn;
         tt[e] = (i == n16 ? 1.f : 0.f) - xt[e];                  // T^T, first factor
       }
-      if constexpr (FULL) sm.mt[wave][1][lane] = Op::a(aq);      // Aq = [j <= i] e^{G_i - G_j} q_i.k_j
+      if constexpr (FULL) sm.mt[wave][1][lane] = aq;      // Aq = [j <= i] e^{G_i - G_j} q_i.k_j
 #pragma unroll
       for (int step = 0; step < 3; ++step) {
         f32x4 s2 = zero4(), s2t = zero4();
-        mma16(s2, Op::a(xt), Op::b(xa));                         // X^2
-        if (step < 2) mma16(s2t, Op::a(xa), Op::b(xt));          // (X^2)^T
-        mma16(tt, Op::a(s2), Op::b(tt));                         // T^T += (X^2)^T T^T
+        mma(s2, xt, xa);                                         // X^2
+        if (step < 2) mma(s2t, xa, xt);                          // (X^2)^T
+        mma(tt, s2, tt);                                         // T^T += (X^2)^T T^T
         xa = s2;
         xt = s2t;
       }
-      sm.mt[wave][0][lane] = Op::a(tt);
-      const typename Op::B tb = Op::b(tt);
+      sm.mt[wave][0][lane] = tt;
       // the window's blocks: the one that sub-chunk c - z wrote last (z = 1 ..
       // NB; c itself writes the last of them), its slot j holding the key of
       // that sub-chunk's token j, or the carried state's key where that token
       // came before this call, decayed from there to c's start
       //   Ho_b = vis alpha_i e^{G_i + off_j} h_i.k_j,  Qo_b = vis e^{G_i + off_j} q_i.k_j,
       // vis: not yet overwritten by sub-chunk c; W_b = T Ho_b
-      const float el = decay_exp<CT>(gl);
+      const float el = expf(gl);
       f32x4 ei;
 #pragma unroll
       for (int e = 0; e < 4; ++e) ei[e] = __shfl(el, 4 * g4 + e, 64);
@@ -392,7 +344,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
           mma(ho, hf[kb], pf[kb]);
           if constexpr (FULL) mma(qt, pf[kb], x.q[kb]);
         }
-        const float eo = decay_exp<CT>(off);
+        const float eo = expf(off);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int i = 4 * g4 + e;
@@ -403,9 +355,9 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
           if constexpr (FULL) qt[e] *= vist ? el * eoi : 0.f;
         }
         f32x4 wt = zero4();
-        mma16(wt, Op::a(ho), tb);                                // W_b^T = Ho_b^T T^T
-        sm.mt[wave][2 + b][lane] = Op::a(-wt);
-        if constexpr (FULL) sm.mt[wave][2 + NB + b][lane] = Op::a(qt);
+        mma(wt, ho, tt);                                         // W_b^T = Ho_b^T T^T
+        sm.mt[wave][2 + b][lane] = -wt;
+        if constexpr (FULL) sm.mt[wave][2 + NB + b][lane] = qt;
       }
     }
     lds_barrier();
@@ -417,8 +369,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       const bool whole = tr >= 0 && tr + kSC <= T;   // (uniform) every token is of this call
       const f32x4 aw = *(const f32x4*)&sm.aw[s][4 * g4], kco = *(const f32x4*)&sm.kco[s][4 * g4];
       const f32x4 qco = *(const f32x4*)&sm.qco[s][4 * g4];
-      const typename Op::A trow = sm.mt[s][0][lane];
-      typename Op::A wrow[NB], qrow[NB], arow;
+      const f32x4 trow = sm.mt[s][0][lane];
+      f32x4 wrow[NB], qrow[NB], arow;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         wrow[b] = sm.mt[s][2 + b][lane];
@@ -455,23 +407,20 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int a = 0; a < TU; ++a) {
         un[a] = zero4();
-        if (a < TPW) mma16(un[a], trow, Op::b(rhs[a < TPW ? a : 0] - kco * kh[a < TPW ? a : 0]));
+        if (a < TPW) mma(un[a], trow, rhs[a < TPW ? a : 0] - kco * kh[a < TPW ? a : 0]);
       }
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int a = 0; a < TU; ++a) mma16(un[a], wrow[b], ub[b][a]);
-      typename Op::B nb[TU];
-#pragma unroll
-      for (int a = 0; a < TU; ++a) nb[a] = Op::b(un[a]);
+        for (int a = 0; a < TU; ++a) mma(un[a], wrow[b], uo[b][a]);
       if constexpr (FULL) {
         f32x4 y[TPW];
 #pragma unroll
         for (int a = 0; a < TPW; ++a) {
           y[a] = qco * kq[a];
 #pragma unroll
-          for (int b = 0; b < NB; ++b) mma16(y[a], qrow[b], ub[b][a]);
-          mma16(y[a], arow, nb[a]);
+          for (int b = 0; b < NB; ++b) mma(y[a], qrow[b], uo[b][a]);
+          mma(y[a], arow, un[a]);
         }
         CT* yp = (CT*)p.y + tk.y_base + (ptrdiff_t)tr * (ptrdiff_t)tk.y_tok;
         const unsigned yo = (unsigned)(4 * g4 * (int)tk.y_tok + wave * TPW * 16 + n16);
@@ -503,10 +452,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (b == beta) {
           if (whole) {
 #pragma unroll
-            for (int a = 0; a < TU; ++a) {
-              uo[b][a] = un[a];
-              ub[b][a] = nb[a];
-            }
+            for (int a = 0; a < TU; ++a) uo[b][a] = un[a];
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -515,8 +461,6 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
                 for (int a = 0; a < TU; ++a) uo[b][a][e] = un[a][e];
             }
-#pragma unroll
-            for (int a = 0; a < TU; ++a) ub[b][a] = Op::b(uo[b][a]);
           }
         }
     }

@@ -2,6 +2,8 @@
 carried from run to run, the state's keys and writes seen across ragged call
 edges, against the CPU oracle (rel-L2 1e-4 in float32, 1e-2 in bf16, the
 net writes twice that, the keys 1e-5)."""
+import math
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -57,3 +59,33 @@ def test_runs_match_oracle(gpu_lib, D, P, Kc, t0, T, io):
     assert rel_l2(y, yr) <= tol
     assert rel_l2(s[2], sr[2]) <= 2 * tol
     assert rel_l2(s[3], sr[3]) <= 1e-5     # keys decay in float32 from the inputs
+
+
+@pytest.mark.parametrize("io", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("P,scale", [(16, 1.0), (16, 2.0), (64, 1.0), (64, 2.0)])
+def test_runs_alike_keys(gpu_lib, P, scale, io):
+    """Keys that are nearly one direction (a repeated token), decay near 1: the
+    powers of L that make up T = (I + L)^-1 cancel.  With l the largest entry
+    of L the factors' entries reach (1 + l)^15 where T's stay below 1, so
+    products in float32 leave up to 2^-24 (1 + l)^15 in the net writes, and
+    16-bit parts of them 2^-17 (1 + l)^15.  b = 1 keeps h = k exact in bf16."""
+    print(f"case: gdn3 runs alike keys P={P} scale={scale} {io}", flush=True)
+    B, T, H, M, D = 1, 133, 1, 2, 128
+    g = torch.Generator().manual_seed(31 + P)
+    base = F.normalize(torch.randn(B, 1, H, D, generator=g), dim=-1)
+    k = (scale * F.normalize(base + 1e-3 * torch.randn(B, T, H, D, generator=g), dim=-1)).to(io)
+    q = F.normalize(base + 0.5 * torch.randn(B, T, H, D, generator=g), dim=-1).to(io)
+    v = (torch.randn(B, 1, H, D, generator=g) + 0.1 * torch.randn(B, T, H, D, generator=g)).to(io)
+    one = torch.ones(B, T, H, M)
+    dec = one * torch.tensor([1.0, 0.999])
+    wide = (B, T, H, M, D)
+    ex = [x.double().unsqueeze(3).expand(wide) for x in (q, k, v)]
+    gx = one.double().unsqueeze(-1).expand(wide)
+    cfg = dict(R=4, P=P, factors=(16, 16, 8, 8), compact_every=1 << 20, return_state=True)
+    yr, sr, _ = og.gdn3_recurrence(*ex, gx, gx, dec.double(), sign_mode="canonical", **cfg)
+    y, s, _ = gdn3.gdn3_recurrent_state(*(x.to(DEV) for x in (q, k, v, one, one, dec)), **cfg)
+    torch.cuda.synchronize()
+    kk = k.double().square().sum(-1).max().item()
+    bound = 2.0 ** -24 * (1 + (1 - math.exp(-kk))) ** 15      # l = alpha(k.k) k.k
+    assert rel_l2(s[2], sr[2]) <= bound
+    assert rel_l2(y, yr) <= bound + (2.0 ** -9 if io == torch.bfloat16 else 0.0)   # y's own rounding

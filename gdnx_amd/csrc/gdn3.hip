@@ -1736,7 +1736,7 @@ int run_gdn3_fwd(G3FwdArgs a, hipStream_t stream) {
 // cannot allocate (graph capture, serving loops).  Each device the library
 // runs on holds its own copy for the life of the process; host code reaches
 // it only through the address hipGetSymbolAddress returns for that device.
-static __device__ __align__(256) unsigned char scratch[kG3ScratchBytes + kG3LongScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kG3ScratchBytes];
 
 namespace {
 std::mutex g_scratch_mu;
@@ -1768,15 +1768,11 @@ int gdn3_zero_fill(float* p, size_t n, hipStream_t stream) {
   return check_launch("fill_zero_kernel");
 }
 
-size_t gdn3_state_bytes(int N, int D, int P, int dtype) {
+size_t gdn3_workspace_bytes(int N, int D, int P, int dtype) {
   const size_t cb = dtype == GDNX_DTYPE_BF16 ? 2 : 4;
   const int R = 4, mn = D == 128 ? 256 + 64 : 64 + 64;
   return align256((size_t)N * D * D * cb) + align256((size_t)N * R * mn * 4) + 2 * align256((size_t)N * P * D * 4) +
-         align256((size_t)N * 4);
-}
-
-size_t gdn3_workspace_bytes(int N, int D, int P, int dtype) {
-  return gdn3_state_bytes(N, D, P, dtype) + gdn3_long_bytes(N, D, P);
+         align256((size_t)N * 4) + gdn3_long_bytes(N, D, P);
 }
 
 size_t gdn3_train_states_bytes(int N, int T, int D, int P, int Kc) {

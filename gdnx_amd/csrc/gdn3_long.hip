@@ -177,8 +177,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
     if constexpr (FULL) {
 #pragma unroll 2
       for (int x = 0; x < r; ++x) {
-        const float* ru = p.run_u + ((size_t)chain * p.nrun + x) * P * D;
-        const float* rv = p.run_v + ((size_t)chain * p.nrun + x) * P * P;
+        const float* ru = p.run_u + ((size_t)chain * (p.nrun - 1) + x) * P * D;
+        const float* rv = p.run_v + ((size_t)chain * (p.nrun - 1) + x) * P * P;
         f32x4 nu[NB][TPW];
 #pragma unroll
         for (int bl = 0; bl < NB; ++bl) {
@@ -469,8 +469,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 
   if constexpr (!FULL) {
-    float* ru = p.run_u + ((size_t)chain * p.nrun + r) * P * D;
-    float* rv = p.run_v + ((size_t)chain * p.nrun + r) * P * P;
+    float* ru = p.run_u + ((size_t)chain * (p.nrun - 1) + r) * P * D;
+    float* rv = p.run_v + ((size_t)chain * (p.nrun - 1) + r) * P * P;
 #pragma unroll
     for (int bl = 0; bl < NB; ++bl)
 #pragma unroll
@@ -571,16 +571,19 @@ int runs_max(int N) { return N >= kG3RunTarget ? 1 : kG3RunTarget / N; }
 
 }  // namespace
 
-// the other copy of the window state and the runs' maps
+// the other copy of the window state and the maps of all runs but the last.
+// At most 256 chains have any: with their states that is 61.3 MiB at d = 128,
+// P = 64, float32, so that the workspace fits the static scratch exactly where
+// the states do.
 size_t gdn3_long_bytes(int N, int D, int P) {
   if (N <= 0 || runs_max(N) == 1) return 0;
-  const size_t n = (size_t)N * runs_max(N);
+  const size_t n = (size_t)N * (runs_max(N) - 1);
   return 2 * g3_align256((size_t)N * P * D * 4) + g3_align256(n * P * D * 4) + g3_align256(n * P * P * 4);
 }
 
 void gdn3_long_carve(G3FwdArgs& a, int N, char* w) {
   if (runs_max(N) == 1) return;
-  const size_t n = (size_t)N * runs_max(N), win = g3_align256((size_t)N * a.P * a.D * 4);
+  const size_t n = (size_t)N * (runs_max(N) - 1), win = g3_align256((size_t)N * a.P * a.D * 4);
   a.uw_alt = (float*)w;
   a.vw_alt = (float*)(w + win);
   a.run_u = (float*)(w + 2 * win);

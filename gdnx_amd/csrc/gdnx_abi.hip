@@ -576,7 +576,7 @@ extern "C" int gdnx_gdn3_chunk_fwd_state_noalloc(const void* q, const void* k, c
   if ((rc = g3_state_check(A0, B0, U0, Vb0, t0, T))) return rc;
   // (the layer's default regime runs as one fused launch and needs no scratch)
   const size_t need = gdn3_fwd_fused(head_dim, P, compact_every, dtype)
-                          ? 0 : gdn3_state_bytes(B * H * M, head_dim, P, dtype);
+                          ? 0 : gdn3_workspace_bytes(B * H * M, head_dim, P, dtype);
   if (need > kG3ScratchBytes)
     return set_error(GDNX_ERR_WORKSPACE,
                      "gdn3 no-alloc forward: %d chains need %zu bytes of scratch; the library's static scratch "

@@ -204,8 +204,8 @@ struct G3FwdArgs {
   float* vw_alt;
   float* uw_out;
   float* vw_out;
-  float* run_u;        // [N, runs, P, D]
-  float* run_v;        // [N, runs, P, P]
+  float* run_u;        // [N, runs - 1, P, D]
+  float* run_v;        // [N, runs - 1, P, P]
   int nrun, rlen;
 };
 
@@ -321,19 +321,13 @@ int gdn3_fwd_dispatch(const G3FwdArgs& a, hipStream_t stream);
 bool gdn3_fwd_fused(int D, int P, int Kc, int dtype);
 // bytes of the static scratch of gdnx_gdn3_chunk_fwd_state_noalloc (per device)
 constexpr size_t kG3ScratchBytes = (size_t)64 << 20;
-// workgroups an interval is spread over (chains x runs),
-// and what that takes at most beside the state (d = 128, P = 64, 256 chains:
-// the other copy of the window state and the maps of 512 runs)
+// workgroups an interval is spread over (chains x runs)
 constexpr int kG3RunTarget = 512;
-constexpr size_t kG3LongScratchBytes = (size_t)48 << 20;
 // that scratch's address on the current device (resolved once per device)
 int gdn3_scratch(void** out);
 // p[0, n) = 0 on the stream (a fill kernel: safe inside graph capture)
 int gdn3_zero_fill(float* p, size_t n, hipStream_t stream);
 size_t gdn3_workspace_bytes(int N, int D, int P, int dtype);
-// of it, what holds the state between launches (the no-alloc entry's limit
-// counts this part)
-size_t gdn3_state_bytes(int N, int D, int P, int dtype);
 // the intervals between compactions (gdn3_long.hip)
 size_t gdn3_long_bytes(int N, int D, int P);
 void gdn3_long_carve(G3FwdArgs& a, int N, char* w);

@@ -358,11 +358,11 @@ int gdnx_gdn3_chunk_fwd_state(const void* q, const void* k, const void* v, int q
  * nothing and takes no caller memory beyond inputs and outputs.  No
  * counterpart in the reference; for callers that cannot allocate (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc).  The
- * workspace lives in a static device array that each GPU the library runs on
- * holds until the process ends: gdnx_gdn3_noalloc_scratch_bytes() bytes (64
- * MiB) for the chains' states and 48 MiB for the runs of long intervals.
- * Calls whose states need more than the first (about 1,250 chains in bf16, 780
- * in float32 at head_dim 128) return GDNX_ERR_WORKSPACE before any launch.  All
+ * workspace lives in a static device array of
+ * gdnx_gdn3_noalloc_scratch_bytes() bytes (64 MiB) that each GPU the library
+ * runs on holds until the process ends; calls needing more
+ * (gdnx_gdn3_workspace_bytes > that: about 1,250 chains in bf16, 780 in
+ * float32 at head_dim 128) return GDNX_ERR_WORKSPACE before any launch.  All
  * calls on one GPU share its array: calls that overlap on one GPU (other
  * streams or threads) race.  Results equal gdnx_gdn3_chunk_fwd_state's. */
 long long gdnx_gdn3_noalloc_scratch_bytes(void);

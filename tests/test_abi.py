@@ -285,6 +285,32 @@ def test_gdn3_decode_step_rejects_negative_positions():
         gdn3.gdn3_decode_step(x, x, x, gates, gates, gates, state, [3, -1], factors=(8, 8, 8, 8))
 
 
+def test_noalloc_scratch_holds_what_its_query_says():
+    """gdnx_gdn3_workspace_bytes > gdnx_gdn3_noalloc_scratch_bytes is the
+    documented test for a call that the entry refuses.  What a workspace holds
+    beside the chains' states (the runs of long intervals) must not move that
+    line: it lies where the states alone (Kronecker matrix, factors, window,
+    log decay, each rounded to 256 bytes) fill the scratch."""
+    from gdnx_amd import _lib
+    lib = _lib.load()
+    cap = lib.gdnx_gdn3_noalloc_scratch_bytes()
+
+    def up(x):
+        return (x + 255) // 256 * 256
+    for D in (64, 128):
+        for P in (16, 32, 64):
+            for dt, cb in ((_lib.DTYPE_BF16, 2), (_lib.DTYPE_F32, 4)):
+                fit = 0
+                for N in range(1, 6000):
+                    state = (up(N * D * D * cb) + up(N * 4 * ((256 if D == 128 else 64) + 64) * 4)
+                             + 2 * up(N * P * D * 4) + up(N * 4))
+                    ws = lib.gdnx_gdn3_workspace_bytes(1, N, 1, D, P, dt)
+                    assert ws >= state
+                    assert (ws <= cap) == (state <= cap), (D, P, dt, N)
+                    fit += ws <= cap
+                assert 0 < fit < 5999
+
+
 def test_noalloc_forward_refuses_before_any_launch():
     """The allocation-free GDN3 forward checks its static scratch's size
     before touching a device: too many chains is GDNX_ERR_WORKSPACE here too."""

@@ -73,3 +73,20 @@ def test_noalloc_forward_equals_workspace_forward(gpu_lib, io, P, Kc):
         for a, b in zip(s, s_ref):
             assert torch.equal(a, b), (B, T)
         assert torch.equal(c, c_ref)
+
+
+@pytest.mark.parametrize("B,T,H,M,t0,P,Kc,io", [
+    (1, 1100, 2, 2, 0, 16, 2048, torch.bfloat16),      # one interval, the most runs of a few chains
+    (1, 1300, 1, 3, 21, 32, 512, torch.bfloat16),      # several intervals of several runs, a ragged start
+    (1, 600, 16, 16, 0, 64, 1024, torch.float32),      # the most chains with runs, their largest workspace
+], ids=["one", "several", "widest"])
+def test_noalloc_forward_over_runs(gpu_lib, B, T, H, M, t0, P, Kc, io):
+    """Long intervals: the runs' maps and the window's other copy in the scratch."""
+    print(f"case: gdn3 no-alloc forward over runs T={T} P={P} Kc={Kc} {io}", flush=True)
+    x, st0 = _inputs(B, T, H, M, 128, 3, io, P)
+    y_ref, s_ref, c_ref = _run(gpu_lib, False, x, st0, t0, B, T, H, M, 128, io, P, Kc)
+    y, s, c = _run(gpu_lib, True, x, st0, t0, B, T, H, M, 128, io, P, Kc)
+    assert torch.isfinite(y.float()).all()
+    assert torch.equal(y, y_ref) and torch.equal(c, c_ref)
+    for a, b in zip(s, s_ref):
+        assert torch.equal(a, b)

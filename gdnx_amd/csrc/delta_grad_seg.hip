@@ -1,6 +1,6 @@
 // Checkpointed gradient kernel of the chunked delta rule (gfx950): the
-// backward's last stage when the forward kept one state per 256-token
-// segment (bf16 IO, 32-token scan chunks, at most 4 lanes per head).
+// backward's last stage when the forward kept one state per segment of 256
+// tokens, or 128 or 64 (bf16 IO, 32-token scan chunks, at most 4 lanes per head).
 //
 // Per chain (b, h, m) and 32-token sub-chunk, with S the state entering the
 // sub-chunk and dS the gradient of the state leaving it (see delta_bwd.hip
@@ -51,7 +51,7 @@ constexpr int kRes = 2;       // lanes whose states are resident at a time
 template <int D>
 struct SegDims {
   static constexpr int C = 32;                           // sub-chunk (tokens)
-  static constexpr int NSUB = kSegTokens / C;            // sub-chunks per segment, at most (p.cps)
+  static constexpr int NSUB = kSegTokens / C;            // sub-chunks per segment, at most
   static constexpr int NW = D / 16;                      // waves; wave w owns key (and value) tile w
   static constexpr int NT = 64 * NW;
   static constexpr int NDT = D / 16;
@@ -164,7 +164,11 @@ __device__ __forceinline__ uint4 nt_load16(const bf16* p) {
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-template <int D>
+// SEG: tokens per segment, which is also what a segment's carry takes (16 heads
+// of one sequence of 1999 tokens, 128 a segment: 50 MB; 101 with room for 256).
+// As a constant: with the carry's distances in registers the kernel was 13 us
+// slower at 64 heads, T = 4096 (808 -> 821).
+template <int D, int SEG>
 __global__ void __launch_bounds__(SegDims<D>::NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 delta_grad_seg_kernel(DeltaBwdArgs p) {
   typedef SegDims<D> Sd;
@@ -182,12 +186,12 @@ delta_grad_seg_kernel(DeltaBwdArgs p) {
   const int BH = p.B * p.H, M = p.M;
   const int s = blockIdx.x / BH, bh = blockIdx.x % BH, b = bh / p.H, h = bh % p.H;
   const int N = BH * M;
-  const int seg = p.cps * C, t_seg = s * seg;   // tokens per segment
-  const int nsub = min(p.cps, (p.T - t_seg + C - 1) / C);
+  const int t_seg = s * SEG;
+  const int nsub = min(SEG / C, (p.T - t_seg + C - 1) / C);
   // the scans' chunk, which is the stash's record length and the sub-chunk
   // (dispatch rejects any other p.C), so record offsets are shifts
   constexpr int CS = C;
-  const StashGeom sg = stash_geom(N, p.T, D, CS, p.cps);
+  const StashGeom sg = stash_geom(N, p.T, D, CS, SEG / CS);
   const bf16* sck = (const bf16*)p.s_stash;   // state records, then the net writes R
   const bf16* rst = sck + sg.states;
   const bf16* dsck = (const bf16*)p.ds_stash; // state-gradient records, then dB, then P3
@@ -196,11 +200,11 @@ delta_grad_seg_kernel(DeltaBwdArgs p) {
   const float* k3st = (const float*)(p3st + sg.tiles);   // k.P3 per token
   // this workgroup's float32 carry of the dq, dk, dv sums from one lane pair
   // to the next, [3][sub-chunk][wave][token tile][64 lanes][4]
-  const int NSEG = (p.T + seg - 1) / seg;
-  float* const dqs = (float*)((char*)p.ds_stash + delta_seg_carry_offset(N, p.T, D, CS, p.cps)) +
-                     ((size_t)bh * NSEG + s) * 3 * kSegTokens * D;
-  float* const dks = dqs + kSegTokens * D;
-  float* const dvs = dqs + 2 * kSegTokens * D;
+  const int NSEG = (p.T + SEG - 1) / SEG;
+  float* const dqs = (float*)((char*)p.ds_stash + delta_seg_carry_offset(N, p.T, D, CS, SEG / CS)) +
+                     ((size_t)bh * NSEG + s) * 3 * SEG * D;
+  float* const dks = dqs + SEG * D;
+  float* const dvs = dqs + 2 * SEG * D;
   const size_t rs = (size_t)p.H * D;                  // q/k/v token stride
   const size_t rsy = (size_t)p.H * M * D;             // dy token stride
   const size_t st = (size_t)p.H * M;                  // scalar token stride
@@ -670,23 +674,26 @@ delta_grad_seg_kernel(DeltaBwdArgs p) {
   }   // lane pairs
 }
 
+template <int D, int SEG = kSegTokens>
+int launch_grad_seg(const DeltaBwdArgs& a, hipStream_t stream) {
+  static_assert(sizeof(SegSmem<D>) <= 160 * 1024, "LDS budget");
+  if constexpr (SEG > 64)
+    if (a.cps * SegDims<D>::C < SEG) return launch_grad_seg<D, SEG / 2>(a, stream);
+  const unsigned grid = (unsigned)(a.B * a.H * ((a.T + SEG - 1) / SEG));
+  hipLaunchKernelGGL((delta_grad_seg_kernel<D, SEG>), dim3(grid), dim3(SegDims<D>::NT), 0, stream, a);
+  return check_launch("delta_grad_seg_kernel");
+}
+
 }  // namespace
 
 int delta_grad_seg_dispatch(const DeltaBwdArgs& a, hipStream_t stream) {
-  if (a.cps < 1 || a.cps > SegDims<128>::NSUB) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: segment of %d chunks", a.cps);
-  const int seg = a.cps * a.C, NSEG = (a.T + seg - 1) / seg;
-  const unsigned grid = (unsigned)(a.B * a.H * NSEG);
   if (a.M > kLaneCap) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: at most %d lanes per head", kLaneCap);
   if (a.C != SegDims<128>::C) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: %d-token chunks only", SegDims<128>::C);
-  if (a.D == 128) {
-    static_assert(sizeof(SegSmem<128>) <= 160 * 1024, "LDS budget");
-    hipLaunchKernelGGL((delta_grad_seg_kernel<128>), dim3(grid), dim3(SegDims<128>::NT), 0, stream, a);
-  } else if (a.D == 64) {
-    hipLaunchKernelGGL((delta_grad_seg_kernel<64>), dim3(grid), dim3(SegDims<64>::NT), 0, stream, a);
-  } else {
-    return set_error(GDNX_ERR_SHAPE, "checkpointed backward: unsupported head dim %d", a.D);
-  }
-  return check_launch("delta_grad_seg_kernel");
+  const int seg = a.cps * a.C;
+  if (seg != 256 && seg != 128 && seg != 64) return set_error(GDNX_ERR_SHAPE, "checkpointed backward: segment of %d tokens", seg);
+  if (a.D == 128) return launch_grad_seg<128>(a, stream);
+  if (a.D == 64) return launch_grad_seg<64>(a, stream);
+  return set_error(GDNX_ERR_SHAPE, "checkpointed backward: unsupported head dim %d", a.D);
 }
 
 }  // namespace gdnx

@@ -46,7 +46,7 @@ size_t delta_bwd_workspace_bytes(int B, int T, int H, int M, int D, int C, int d
   if (cps > 1) {   // see delta_seg_carry_offset
     const size_t seg = (size_t)cps * C, nseg = ((size_t)T + seg - 1) / seg;
     return delta_seg_carry_offset(B * H * M, T, D, C, cps) +
-           (M > 2 ? 3 * (size_t)B * H * nseg * kSegTokens * D * sizeof(float) : 0);
+           (M > 2 ? 3 * (size_t)B * H * nseg * seg * D * sizeof(float) : 0);
   }
   size_t n = delta_stash_bytes(B * H * M, T, D, C, dtype, cps);
   if (dtype == GDNX_DTYPE_BF16 && C == 64) {

@@ -383,7 +383,7 @@ __host__ __device__ inline StashGeom stash_geom(int nchains, int T, int D, int C
 // The checkpointed backward's workspace (bf16 IO): the state gradients at
 // segment ends, dB and P3 = R dS^T per token (bf16), k.P3 per token
 // (float32), then, with more than two lanes per head, the float32 carry of
-// the dq / dk / dv sums between lane pairs ([B H segments][3][kSegTokens][D]).
+// the dq / dk / dv sums between lane pairs ([B H segments][3][tokens per segment][D]).
 __host__ __device__ inline size_t delta_seg_carry_offset(int nchains, int T, int D, int C, int cps) {
   const StashGeom g = stash_geom(nchains, T, D, C, cps);
   return ((g.states + 2 * g.tiles) * 2 + g.nrec * C * sizeof(float) + 255) / 256 * 256;
@@ -395,7 +395,7 @@ inline size_t delta_stash_bytes(int nchains, int T, int D, int C, int dtype, int
 }
 // bytes of the backward's workspace: state gradients and dB like the
 // forward's stash, then (checkpointed form) the gradient kernel's float32
-// dq / dk / dv sums, [B, H, segments][3][kSegTokens][D], or (64-token
+// dq / dk / dv sums, [B, H, segments][3][tokens per segment][D], or (64-token
 // chunks in the per-chunk form) the key halves' per-token partials
 size_t delta_bwd_workspace_bytes(int B, int T, int H, int M, int D, int C, int dtype);
 int delta_bwd_dispatch(const DeltaBwdArgs& a, int stages, hipStream_t stream);

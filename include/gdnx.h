@@ -85,7 +85,7 @@ long long gdnx_delta_chunk_states_bytes(int B, int T, int H, int M, int head_dim
  * the checkpointed form then P3 = R dS^T of every chunk (bf16, the gradient
  * kernel's dk tile layout) and k.P3 per token (float32), and with more than
  * two lanes per head the gradient kernel's float32 carry of the dq, dk and dv
- * sums between lane pairs, 3 x 256 x head_dim floats per (batch, head,
+ * sums between lane pairs, 3 x tokens x head_dim floats per (batch, head,
  * segment).  Changed in ABI 12 (P3 and k.P3 added): query it, do not cache
  * sizes across versions. */
 long long gdnx_delta_bwd_workspace_bytes(int B, int T, int H, int M, int head_dim, int chunk,

@@ -60,6 +60,12 @@ def test_abi_version_and_sizes():
         (ckpt + 255) // 256 * 256 + 3 * 4 * 16 * nseg * 256 * 128 * 4
     ckpt2 = 4 * 16 * 2 * ((nseg * 128 * 128 + 2 * 128 * 32 * 128) * 2 + 128 * 32 * 4)
     assert lib.gdnx_delta_bwd_workspace_bytes(4, 4096, 16, 2, 128, 32, _lib.DTYPE_BF16) == (ckpt2 + 255) // 256 * 256
+    # few heads or tokens: segments of 128 or 64 tokens, the carry of as many
+    for BH, T, seg in ((16, 1999, 128), (4, 1000, 64), (2, 40, 64)):
+        nseg, nch = -(-T // seg), -(-T // 32)
+        ckpt = BH * 4 * ((nseg * 128 * 128 + 2 * nch * 32 * 128) * 2 + nch * 32 * 4)
+        assert lib.gdnx_delta_bwd_workspace_bytes(1, T, BH, 4, 128, 32, _lib.DTYPE_BF16) == \
+            (ckpt + 255) // 256 * 256 + 3 * BH * nseg * seg * 128 * 4
     # more than 4 lanes: the per-chunk form with its key-half partials
     assert lib.gdnx_delta_bwd_workspace_bytes(1, 128, 1, 5, 128, 64, _lib.DTYPE_BF16) == \
         5 * 2 * (128 * 128 + 64 * 128) * 2 + 2 * 3 * 128 * 5 * 4

@@ -1458,6 +1458,13 @@ __device__ __forceinline__ void compact_chain(const G3CompactArgs& p, G3CompactS
   if (p.skron) write_skron<D, CT>((CT*)p.skron + (size_t)chain * D * D, sm.ab, sm.ab + Rm, tid);
 }
 
+// A decode batch's positions are read this many rows at a time, four a thread
+// in flight (16384 rows of one chain, d = 64, none due: the step 143 us with
+// batches of 256, 73 so, 63 with each workgroup checking its own rows only; 1024
+// due of them 193, 124, 708).
+constexpr int kRowsPer = 4, kRowBatch = 16 * kNT;
+static_assert(kRowBatch / 64 == 64, "a lane per 64 rows of a batch");
+
 template <int D, int P, typename CT>
 __global__ void __launch_bounds__(kNT) gdn3_compact_kernel(G3CompactArgs p) {
   __shared__ G3CompactSmem<D, P> sm;
@@ -1475,40 +1482,49 @@ __global__ void __launch_bounds__(kNT) gdn3_compact_kernel(G3CompactArgs p) {
   // 1024 due chains of 16384 take 4 each on 256 workgroups, 125 us at d =
   // 128 (each workgroup checking its own stride of the chains left all 8 of
   // a stride to one workgroup whenever the rows' positions repeat with a
-  // period that divides it: 220 us).  A step that closes no interval costs
-  // one round of position reads.
-  __shared__ int rows[kNT];
-  __shared__ int wcnt[kNT / 64];
+  // period that divides it: 220 us).
+  __shared__ unsigned short rows[kRowBatch];               // of the batch at base
+  __shared__ unsigned long long mask[kRowBatch / 64];      // due rows by groups of 64
   const int NS = p.N / p.hm, lane = tid & 63, wave = tid >> 6;
-  long long seen = 0;   // due chains of the rows before this batch
-  for (int base = 0; base < NS; base += kNT) {
-    const int row = base + tid;
-    bool go = false;
-    if (row < NS) {
-      const int pos = p.pos[row];
-      go = pos >= 0 && (pos + 1) % p.Kc == 0;   // (a negative position is an empty row)
-      if (go && p.slots) {
-        const int sl = p.slots[row];
-        go = sl >= 0 && sl < p.nslots;
+  const unsigned G = gridDim.x;
+  unsigned seen = 0;   // due chains of the rows before this batch
+  for (int base = 0; base < NS; base += kRowBatch) {
+    const int th = opaque(tid);   // (its address arithmetic is not held across the compactions)
+    const int ng = min(kRowBatch / 64, (NS - base + 63) / 64);   // groups of 64 rows
+#pragma unroll 1
+    for (int j = 0; j * (kNT / 64) < ng; j += kRowsPer) {
+      int ps[kRowsPer], sl[kRowsPer];
+#pragma unroll
+      for (int i = 0; i < kRowsPer; ++i) ps[i] = p.pos[min(base + (j + i) * kNT + th, NS - 1)];
+#pragma unroll
+      for (int i = 0; i < kRowsPer; ++i) sl[i] = p.slots ? p.slots[min(base + (j + i) * kNT + th, NS - 1)] : 0;
+#pragma unroll
+      for (int i = 0; i < kRowsPer; ++i) {
+        const int row = base + (j + i) * kNT + th;
+        if (base + (j + i) * kNT >= NS) break;   // (uniform)
+        const bool go = row < NS && ps[i] >= 0 && (ps[i] + 1) % p.Kc == 0 &&   // (a negative position is an empty row)
+                        (!p.slots || (sl[i] >= 0 && sl[i] < p.nslots));
+        const unsigned long long m = __ballot(go);
+        if (lane == 0) mask[(j + i) * (kNT / 64) + wave] = m;
       }
     }
-    const unsigned long long due = __ballot(go);
-    if (lane == 0) wcnt[wave] = __popcll(due);
     __syncthreads();
-    int at = __popcll(due & ((1ull << lane) - 1)), n = 0;
-#pragma unroll
-    for (int w = 0; w < kNT / 64; ++w) {
-      if (w < wave) at += wcnt[w];
-      n += wcnt[w];
+    // due rows up to group `lane`, inclusive (whole numbers below 2^24)
+    const float upto = lane_prefix<64>(lane < ng ? (float)__popcll(mask[lane]) : 0.f, lane);
+    const unsigned cnt = (unsigned)lane_value(upto, 63) * p.hm;
+    if (cnt) {   // (uniform)
+#pragma unroll 1
+      for (int g = wave; g < ng; g += kNT / 64) {
+        const unsigned long long m = mask[g];
+        const int at = (int)__shfl(upto, g, 64) - __popcll(m) + __popcll(m & ((1ull << lane) - 1));
+        if (m >> lane & 1) rows[at] = (unsigned short)(g * 64 + lane);
+      }
+      __syncthreads();
     }
-    if (go) rows[at] = row;
-    __syncthreads();
-    const long long cnt = (long long)n * p.hm;
-    const int G = gridDim.x;
-    for (long long e = (blockIdx.x + G - seen % G) % G; e < cnt; e += G) {   // due chain seen + e is this workgroup's
-      const int r = rows[e / p.hm], ch = (int)(e % p.hm);
+    for (unsigned e = (blockIdx.x + G - seen % G) % G; e < cnt; e += G) {   // due chain seen + e is this workgroup's
+      const int r = base + rows[e / p.hm], ch = (int)(e % p.hm);
       compact_chain<D, P, CT>(p, sm, (p.slots ? p.slots[r] : r) * p.hm + ch, r * p.hm + ch, tid);
-      __syncthreads();   // the chain's last LDS reads before the next one's loads
+      lds_barrier();   // the chain's last LDS reads before the next one's loads (its stores need not have arrived)
     }
     seen += cnt;
     __syncthreads();   // rows and wcnt are read before the next batch writes them
@@ -1598,28 +1614,41 @@ __global__ void __launch_bounds__(kNT) kron_read_kernel(KronReadArgs p) {
 }
 
 int cu_count() {
-  static int n = 0;
-  if (n == 0) {
+  static const int n = [] {
     int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) ==
-                                                hipSuccess && v > 0)
-      n = v;
-    else
-      n = 256;
-  }
+    return hipGetDevice(&dev) == hipSuccess &&
+                   hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0
+               ? v
+               : 256;
+  }();
   return n;
+}
+
+// A decode batch's due chains go round the workgroups that run at once, one a
+// CU at d = 128 (LDS), two at d = 64 (registers; LDS alone would take three,
+// and with 768 workgroups the last 256 began when the first 512 had done their
+// share: 64 rows x 64 chains all due 229 us a step, 191 so).
+template <int D, int P, typename CT>
+int launch_compact_ct(const G3CompactArgs& a, hipStream_t stream) {
+  int grid = a.N;
+  if (a.pos) {
+    static const int per_cu = [] {
+      int v = 0;
+      return hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, gdn3_compact_kernel<D, P, CT>, kNT, 0) == hipSuccess && v > 0
+                 ? v
+                 : 1;
+    }();
+    const long long fit = (long long)cu_count() * per_cu;
+    if (fit < grid) grid = (int)fit;
+  }
+  hipLaunchKernelGGL((gdn3_compact_kernel<D, P, CT>), dim3(grid), dim3(kNT), 0, stream, a);
+  return check_launch("gdn3_compact_kernel");
 }
 
 template <int D, int P>
 int launch_compact(const G3CompactArgs& a, hipStream_t stream) {
-  // a decode batch's due chains go round the workgroups that LDS lets run at once
-  const long long fit = (long long)cu_count() * (160 * 1024 / (int)sizeof(G3CompactSmem<D, P>));
-  const int grid = a.pos ? (int)(a.N < fit ? a.N : fit) : a.N;
-  if (a.skron && a.skron_dtype == GDNX_DTYPE_BF16)
-    hipLaunchKernelGGL((gdn3_compact_kernel<D, P, bf16>), dim3(grid), dim3(kNT), 0, stream, a);
-  else
-    hipLaunchKernelGGL((gdn3_compact_kernel<D, P, float>), dim3(grid), dim3(kNT), 0, stream, a);
-  return check_launch("gdn3_compact_kernel");
+  return a.skron && a.skron_dtype == GDNX_DTYPE_BF16 ? launch_compact_ct<D, P, bf16>(a, stream)
+                                                     : launch_compact_ct<D, P, float>(a, stream);
 }
 
 int compact_dispatch(const G3CompactArgs& a, hipStream_t stream) {

@@ -46,3 +46,40 @@ def test_decode_due_rows_spread_over_workgroups(gpu_lib):
     gdn3.gdn3_decode_step(q, k, v, b, w, dec, plain, ps, R=R, P=P, factors=f, compact_every=1 << 20, slots=sl)
     changed = (batch[0] != plain[0]).flatten(1).any(1).nonzero()[:, 0].tolist()
     assert sorted(rows) == changed
+
+
+@pytest.mark.parametrize("NS", [4095, 4097, 8500])
+def test_decode_due_rows_beyond_one_batch(gpu_lib, NS):
+    """More rows than are listed at once (4096), with and without slots: the
+    same as the rows stepped a hundred and one at a time, bitwise."""
+    print(f"case: decode due rows, {NS} rows", flush=True)
+    H, M, D, P, Kc, R, f = 1, 1, 64, 16, 16, 4, (8, 8, 8, 8)
+    g = torch.Generator().manual_seed(NS)
+    pos = torch.randint(0, 64, (NS,), generator=g).to(torch.int32)
+    state = [torch.randn(NS, H, M, *s, generator=g) * 0.2 for s in ((R, 8, 8), (R, 8, 8), (D, P), (D, P))]
+    q, k, v = (torch.nn.functional.normalize(torch.randn(NS, H, D, generator=g), dim=-1).bfloat16().to(DEV)
+               for _ in range(3))
+    b, w = (torch.rand(NS, H, M, generator=g).to(DEV) for _ in range(2))
+    dec = (0.9 + 0.1 * torch.rand(NS, H, M, generator=g)).to(DEV)
+    ps = pos.to(DEV)
+    for slots in (None, torch.randperm(NS, generator=g).to(torch.int32).to(DEV)):
+        batch, parts = [t.to(DEV) for t in state], [t.to(DEV) for t in state]
+        kw = dict(R=R, P=P, factors=f, compact_every=Kc)
+        y = gdn3.gdn3_decode_step(q, k, v, b, w, dec, batch, ps, slots=slots, **kw)
+        ys = []
+        for i in range(0, NS, 101):
+            c = slice(i, i + 101)
+            st = parts if slots is not None else [t[c] for t in parts]
+            ys.append(gdn3.gdn3_decode_step(q[c], k[c], v[c], b[c], w[c], dec[c], st, ps[c],
+                                            slots=None if slots is None else slots[c], sketch=_sketch(c, slots, NS),
+                                            **kw))
+        torch.cuda.synchronize()
+        assert torch.equal(y, torch.cat(ys))
+        for a, e in zip(batch, parts):
+            assert torch.equal(a, e)
+
+
+def _sketch(c, slots, NS):
+    """The sketch rows of the states that a call sees."""
+    G = gdn3.default_sketch(NS, 64, 8, torch.device(DEV))
+    return G if slots is not None else G[c]

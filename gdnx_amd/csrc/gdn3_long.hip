@@ -35,6 +35,7 @@
 // 16, 4 lanes, d = 128, bf16, a compaction every 2048 tokens (64 chains, 8
 // runs), against the walk of the sub-chunks one by one on 8 workgroups per chain
 // that this replaced: the call 5.24 -> 2.14 ms.
+#include <type_traits>
 #include <utility>
 
 #include "gdn3_common.hpp"
@@ -45,14 +46,23 @@ namespace {
 
 constexpr int kBatch = 4;   // sub-chunks a workgroup prepares at once, one per wave
 
-template <typename CT, int D, int P>
+// Where per-channel write gates go: into u = w o v, kept as float32 rows in
+// place of V's, their loads ahead with the rows', unless those rows would
+// leave LDS (and registers) for one workgroup a CU where two are wanted: bf16, d = 128, all
+// value columns in one workgroup.  There they are read inside the step.
+template <typename CT, int D, int NVS>
+constexpr bool kGatesAhead = sizeof(CT) == 4 || D == 64 || NVS == 2;
+
+template <typename CT, int D, int P, int GL, int NVS>
 struct G3RunSmem {
   static constexpr int NB = P / kSC, KB = D / FragT<CT>::KSTEP;
+  static constexpr bool AHEAD = GL == 2 && kGatesAhead<CT, D, NVS>;
   typedef typename FragT<CT>::type Frag;
+  typedef typename std::conditional<AHEAD, float, CT>::type VT;
   Frag hx[kBatch][KB][64];                                  // H rows of the batch as A fragments
   Frag qx[kBatch][KB][64];                                  // Q rows
   f32x4 mt[kBatch][2 + 2 * NB][64];                         // T, Aq, -W_b, Qo_b as A operands
-  alignas(16) CT vx[kBatch][kSC][D + 8];                    // V rows
+  alignas(16) VT vx[kBatch][kSC][D / NVS + (sizeof(VT) == 4 ? 4 : 8)];   // V rows (AHEAD: u), this workgroup's columns
   alignas(16) float aw[kBatch][kSC];                        // alpha w (per-channel gates: alpha)
   alignas(16) float kco[kBatch][kSC], qco[kBatch][kSC];     // alpha e^{2 (Gacc + G)}, e^{2 (Gacc + G)}
   float red[kNT / 64];
@@ -60,13 +70,16 @@ struct G3RunSmem {
 };
 
 // GL: gate layout (1: a scalar per lane, 2: per channel).  FULL: pass 2.
-template <typename CT, int D, int P, int GL, bool FULL>
+// NVS: workgroups a run's value columns go to (2 while each still has a CU).
+template <typename CT, int D, int P, int GL, bool FULL, int NVS>
 __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))) gdn3_run_kernel(G3FwdArgs p) {
-  typedef G3RunSmem<CT, D, P> Sm;
+  typedef G3RunSmem<CT, D, P, GL, NVS> Sm;
   typedef typename FragT<CT>::type Frag;
   typedef G3D<D> Ge;
   constexpr int NB = Sm::NB, KS = FragT<CT>::KSTEP, KB = Sm::KB, EPL = KS / 4;   // elements a lane holds of a k-step
-  constexpr int TPW = D / 64;                                                     // value tiles per wave
+  constexpr int DV = D / NVS, TPW = DV / 64, VK = KB / NVS;   // value columns, tiles per wave, k-steps of a V row
+  constexpr bool AHEAD = Sm::AHEAD;
+  static_assert(TPW >= 1 && VK * KS == DV, "whole tiles and k-steps");
   static_assert(sizeof(Frag) == 16 && EPL * sizeof(CT) == 16, "a fragment is one 16-byte load");
   static_assert(NB >= 1 && NB <= kBatch && D % 64 == 0, "the decay window holds the last four sub-chunks");
   __shared__ Sm sm;
@@ -76,7 +89,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int T = p.T, t0 = p.t0, M = p.M;
   const int nr = FULL ? p.nrun : p.nrun - 1;
   // the lanes of a head's run, which share q, k and v, are neighbours on an XCD
-  const int work = xcd_remap(blockIdx.x, p.B * p.H * M * nr);
+  const int bw = xcd_remap(blockIdx.x, p.B * p.H * M * nr * NVS);
+  const int vs = bw % NVS, work = bw / NVS, vt0 = (DV / 16) * vs;   // value tiles vt0 + [0, DV / 16)
   const int r = (work / M) % nr, chain = (work / M / nr) * M + work % M;
   const int cs = p.c0 + r * p.rlen, ce = min(cs + p.rlen, p.c1);
   const int tlo = max(t0, kSC * p.c0);   // the first token after the state uw, vw stand for
@@ -101,15 +115,19 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   // of row n16 per k-step (rows outside the call read an end row and are
   // zeroed where they are used), each row at a 32-bit offset from a uniform base
   struct Rows {
-    Frag k[KB], q[KB], v[KB], pk[NB == 1 ? KB : 1];
+    Frag k[KB], q[KB], v[VK], pk[NB == 1 ? KB : 1];
+    f32x4 bg[AHEAD ? D / 16 : 1], wg[AHEAD ? DV / 16 : 1];   // per-channel gates
     float d, dp[NB], b, w;
   };
-  auto load_rows = [&](const CT* base, int tr, Frag* dst) {
+  auto load_steps = [&](const CT* base, int tr, Frag* dst, auto steps) {
     const int tb = min(max(tr, 0), T - 1);
     const unsigned off = (unsigned)((min(max(tr + n16, 0), T - 1) - tb) * (int)tk.qkv_tok + g4 * EPL);
     const CT* src = base + (size_t)tb * tk.qkv_tok;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) dst[kb] = *(const Frag*)(src + off + kb * KS);
+    for (int kb = 0; kb < steps(); ++kb) dst[kb] = *(const Frag*)(src + off + kb * KS);
+  };
+  auto load_rows = [&](const CT* base, int tr, Frag* dst) {
+    load_steps(base, tr, dst, std::integral_constant<int, KB>());
   };
   auto dec_at = [&](int tau) {
     return p.dec[tk.dec_base + (size_t)min(max(tau - t0, 0), T - 1) * tk.dec_tok];
@@ -118,8 +136,19 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int tr = kSC * (cb + wave) - t0;
     load_rows(kin, tr, x.k);
     if constexpr (FULL) load_rows(qin, tr, x.q);
-    load_rows(vin, tr, x.v);
+    load_steps(vin + DV * vs, tr, x.v, std::integral_constant<int, VK>());
     if constexpr (NB == 1) load_rows(kin, tr - kSC, x.pk);
+    if constexpr (AHEAD) {
+      const size_t go = tk.gate_base + (size_t)min(max(tr + n16, 0), T - 1) * tk.gate_tok + g4 * EPL;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int e = 0; e < EPL; e += 4) x.bg[(kb * EPL + e) / 4] = *(const f32x4*)(p.bg + go + kb * KS + e);
+#pragma unroll
+      for (int kb = 0; kb < VK; ++kb)
+#pragma unroll
+        for (int e = 0; e < EPL; e += 4) x.wg[(kb * EPL + e) / 4] = *(const f32x4*)(p.wg + go + DV * vs + kb * KS + e);
+    }
     x.d = dec_at(kSC * cb + lane);
 #pragma unroll
     for (int z = 0; z < NB; ++z) x.dp[z] = dec_at(kSC * (cb + wave - 1 - z) + n16);
@@ -144,7 +173,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int a = 0; a < TPW; ++a)
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
-        sk[a][kb] = *(const Frag*)((const CT*)p.skron + ((size_t)chain * D + (wave * TPW + a) * 16 + n16) * D + kb * KS +
+        sk[a][kb] = *(const Frag*)((const CT*)p.skron + ((size_t)chain * D + (vt0 + wave * TPW + a) * 16 + n16) * D + kb * KS +
                                    g4 * EPL);
 
   // the window's net writes: [block][tile], the tiles past TPW (pass 1) the
@@ -158,7 +187,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       uo[bl][a] = zero4();
       if (FULL && !p.first)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) uo[bl][a][e] = uw[(bl * kSC + 4 * g4 + e) * D + (wave * TPW + a) * 16 + n16];
+        for (int e = 0; e < 4; ++e) uo[bl][a][e] = uw[(bl * kSC + 4 * g4 + e) * D + (vt0 + wave * TPW + a) * 16 + n16];
     }
     if constexpr (!FULL)
 #pragma unroll
@@ -188,7 +217,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
           for (int a = 0; a < TPW; ++a)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) nu[bl][a][e] = ru[(bl * kSC + 4 * g4 + e) * D + (wave * TPW + a) * 16 + n16];
+            for (int e = 0; e < 4; ++e) nu[bl][a][e] = ru[(bl * kSC + 4 * g4 + e) * D + (vt0 + wave * TPW + a) * 16 + n16];
 #pragma unroll
           for (int b2 = 0; b2 < NB; ++b2)
 #pragma unroll
@@ -223,7 +252,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
           for (int e = 0; e < EPL; ++e) {
             x.k[kb][e] = ok ? x.k[kb][e] : from_f<CT>(0.f);
-            x.v[kb][e] = ok ? x.v[kb][e] : from_f<CT>(0.f);
+            if (kb < VK) x.v[kb < VK ? kb : 0][e] = ok ? x.v[kb < VK ? kb : 0][e] : from_f<CT>(0.f);
             if constexpr (FULL) x.q[kb][e] = ok ? x.q[kb][e] : from_f<CT>(0.f);
           }
       }
@@ -238,7 +267,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
           for (int e = 0; e < EPL; e += 4) {
             f32x4 b4 = {x.b, x.b, x.b, x.b};
-            if constexpr (GL == 2) b4 = *(const f32x4*)(bp + kb * KS + e);
+            if constexpr (AHEAD) b4 = x.bg[(kb * EPL + e) / 4];
+            else if constexpr (GL == 2) b4 = *(const f32x4*)(bp + kb * KS + e);
 #pragma unroll
             for (int i = 0; i < 4; ++i) bb[e + i] = b4[i];
           }
@@ -250,7 +280,21 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
           }
           sm.hx[wave][kb][lane] = hf[kb];
           if constexpr (FULL) sm.qx[wave][kb][lane] = x.q[kb];
-          *(Frag*)&sm.vx[wave][n16][kb * KS + g4 * EPL] = x.v[kb];
+          if (kb < VK) {
+            const Frag vr = x.v[kb < VK ? kb : 0];
+            typename Sm::VT* dst = &sm.vx[wave][n16][kb * KS + g4 * EPL];
+            if constexpr (AHEAD) {
+#pragma unroll
+              for (int e = 0; e < EPL; e += 4) {
+                f32x4 u;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) u[i] = x.wg[kb < VK ? (kb * EPL + e) / 4 : 0][i] * to_f(vr[e + i]);
+                *(f32x4*)(dst + e) = u;
+              }
+            } else {
+              *(Frag*)dst = vr;
+            }
+          }
         }
       }
       const float alpha_l = stable_alpha_f(sum_rows4(part));   // of token n16
@@ -264,7 +308,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
         sm.kco[wave][lane] = alpha_l * e2;
         sm.qco[wave][lane] = e2;
       }
-      if (FULL && p.ts_g && lane == 0) p.ts_g[(size_t)chain * p.nch + c] = gw;
+      if (FULL && p.ts_g && lane == 0 && vs == 0) p.ts_g[(size_t)chain * p.nch + c] = gw;
       // The 16 x 16 matrices.  A product's accumulator tile (row 4 g + e,
       // column n16) is a B operand as it is, and the A operand of its transpose;
       // so a matrix that is wanted as an A operand is formed transposed, by
@@ -382,10 +426,10 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int a = 0; a < TPW; ++a)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int v = (wave * TPW + a) * 16 + n16;
+          const int v = (wave * TPW + a) * 16 + n16;   // of this workgroup's columns
           float wv = 1.f;
-          if constexpr (GL == 2)
-            wv = p.wg[tk.gate_base + (size_t)min(max(tr + 4 * g4 + e, 0), T - 1) * tk.gate_tok + v];
+          if constexpr (GL == 2 && !AHEAD)
+            wv = p.wg[tk.gate_base + (size_t)min(max(tr + 4 * g4 + e, 0), T - 1) * tk.gate_tok + vt0 * 16 + v];
           rhs[a][e] = aw[e] * (wv * to_f(sm.vx[s][4 * g4 + e][v]));
         }
       f32x4 kh[TPW], kq[TPW];
@@ -423,7 +467,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
           mma(y[a], arow, un[a]);
         }
         CT* yp = (CT*)p.y + tk.y_base + (ptrdiff_t)tr * (ptrdiff_t)tk.y_tok;
-        const unsigned yo = (unsigned)(4 * g4 * (int)tk.y_tok + wave * TPW * 16 + n16);
+        const unsigned yo = (unsigned)(4 * g4 * (int)tk.y_tok + (vt0 + wave * TPW) * 16 + n16);
         if (whole) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -439,7 +483,7 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
           }
         }
         if (p.ts_u) {   // training stash: the sub-chunk's net writes
-          float* us = p.ts_u + ((size_t)chain * p.nch + cc) * kSC * D + wave * TPW * 16 + n16;
+          float* us = p.ts_u + ((size_t)chain * p.nch + cc) * kSC * D + (vt0 + wave * TPW) * 16 + n16;
 #pragma unroll
           for (int a = 0; a < TPW; ++a)
 #pragma unroll
@@ -477,8 +521,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int e = 0; e < 4; ++e) {
         const int i = bl * kSC + 4 * g4 + e;
 #pragma unroll
-        for (int a = 0; a < TPW; ++a) ru[i * D + (wave * TPW + a) * 16 + n16] = uo[bl][a][e];
-        if (wave < NB) rv[i * P + wave * kSC + n16] = uo[bl][TPW][e];
+        for (int a = 0; a < TPW; ++a) ru[i * D + (vt0 + wave * TPW + a) * 16 + n16] = uo[bl][a][e];
+        if (wave < NB && vs == 0) rv[i * P + wave * kSC + n16] = uo[bl][TPW][e];
       }
     return;
   } else {
@@ -490,10 +534,11 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int a = 0; a < TPW; ++a)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int i = bl * kSC + 4 * g4 + e, v = (wave * TPW + a) * 16 + n16;
+          const int i = bl * kSC + 4 * g4 + e, v = (vt0 + wave * TPW + a) * 16 + n16;
           p.uw_out[((size_t)chain * P + i) * D + v] = uo[bl][a][e];
           if (p.last && p.U_out) p.U_out[((size_t)chain * D + v) * P + i] = uo[bl][a][e];
         }
+    if (vs > 0) return;   // (what follows is the chain's, not the columns')
     for (int e = tid; e < P * D / EPL; e += kNT) {   // 16 bytes of a slot's key
       const int s = e / (D / EPL), d = EPL * (e % (D / EPL)), b = s / kSC;
       int tau = kSC * (p.c1 - 1 - (p.c1 - 1 - b + kBatch * NB) % NB) + s % kSC;   // the slot's last writer
@@ -533,21 +578,31 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
-template <typename CT, int D, int P, int GL>
+// The value columns of a run on two workgroups while that gives every
+// workgroup a CU of its own.  64 chains, T = 4096, d = 128, a compaction every 64
+// tokens, one workgroup | two (with per-channel gates ahead) | the walk on 8:
+// bf16 2.55 | 2.44 | 2.71 ms, per-channel gates 2.79 | 2.57 | 2.79, float32 3.32 |
+// 2.95 | 3.19, with them 3.54 | 3.06 | 3.27.
+bool value_split(int D, int N, int nrun) { return D == 128 && (long long)N * nrun <= 128; }
+
+template <typename CT, int D, int P, int GL, int NVS>
 int launch_runs(const G3FwdArgs& a, int N, hipStream_t stream) {
-  static_assert(sizeof(G3RunSmem<CT, D, P>) <= 160 * 1024, "LDS budget");
+  static_assert(sizeof(G3RunSmem<CT, D, P, GL, NVS>) <= 160 * 1024, "LDS budget");
   if (a.nrun > 1) {
-    hipLaunchKernelGGL((gdn3_run_kernel<CT, D, P, GL, false>), dim3(N * (a.nrun - 1)), dim3(kNT), 0, stream, a);
+    hipLaunchKernelGGL((gdn3_run_kernel<CT, D, P, GL, false, NVS>), dim3(N * (a.nrun - 1) * NVS), dim3(kNT), 0, stream, a);
     const int rc = check_launch("gdn3_run_kernel");
     if (rc) return rc;
   }
-  hipLaunchKernelGGL((gdn3_run_kernel<CT, D, P, GL, true>), dim3(N * a.nrun), dim3(kNT), 0, stream, a);
+  hipLaunchKernelGGL((gdn3_run_kernel<CT, D, P, GL, true, NVS>), dim3(N * a.nrun * NVS), dim3(kNT), 0, stream, a);
   return check_launch("gdn3_run_kernel");
 }
 
 template <typename CT, int D, int P>
 int launch_runs_gl(const G3FwdArgs& a, int N, hipStream_t stream) {
-  return a.gate_ch > 1 ? launch_runs<CT, D, P, 2>(a, N, stream) : launch_runs<CT, D, P, 1>(a, N, stream);
+  if constexpr (D == 128)
+    if (value_split(a.D, N, a.nrun))
+      return a.gate_ch > 1 ? launch_runs<CT, D, P, 2, 2>(a, N, stream) : launch_runs<CT, D, P, 1, 2>(a, N, stream);
+  return a.gate_ch > 1 ? launch_runs<CT, D, P, 2, 1>(a, N, stream) : launch_runs<CT, D, P, 1, 1>(a, N, stream);
 }
 
 template <typename CT>
@@ -590,10 +645,10 @@ void gdn3_long_carve(G3FwdArgs& a, int N, char* w) {
   a.run_v = (float*)(w + 2 * win + g3_align256(n * a.P * a.D * 4));
 }
 
-// One interval [c0, c1).  With several runs the
-// window state is read from a.uw / a.vw by all of them and left in the other
-// copy (a.uw_alt / a.vw_alt), which then takes a.uw / a.vw's place; a single
-// run updates it in place.
+// One interval [c0, c1).  With several workgroups a chain the window state is
+// read from a.uw / a.vw by all of them and left in the other copy (a.uw_alt /
+// a.vw_alt), which then takes a.uw / a.vw's place; a single one updates it in
+// place.
 int gdn3_long_interval(G3FwdArgs& a, int N, hipStream_t stream) {
   const int nsub = a.c1 - a.c0;
   int nrun = runs_max(N);
@@ -601,11 +656,13 @@ int gdn3_long_interval(G3FwdArgs& a, int N, hipStream_t stream) {
   if (nrun < 1) nrun = 1;
   a.rlen = ((nsub + nrun - 1) / nrun + kBatch - 1) / kBatch * kBatch;
   a.nrun = (nsub + a.rlen - 1) / a.rlen;
-  a.uw_out = a.nrun > 1 ? a.uw_alt : a.uw;
-  a.vw_out = a.nrun > 1 ? a.vw_alt : a.vw;
+  // (two workgroups of a chain read its window as one that may have ended has left it)
+  const bool alt = a.nrun > 1 || value_split(a.D, N, a.nrun);
+  a.uw_out = alt ? a.uw_alt : a.uw;
+  a.vw_out = alt ? a.vw_alt : a.vw;
   const int rc = a.dtype == GDNX_DTYPE_BF16 ? launch_runs_shape<bf16>(a, N, stream)
                                             : launch_runs_shape<float>(a, N, stream);
-  if (a.nrun > 1) {
+  if (alt) {
     std::swap(a.uw, a.uw_alt);
     std::swap(a.vw, a.vw_alt);
   }

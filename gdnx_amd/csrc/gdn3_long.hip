@@ -578,15 +578,8 @@ __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
-// The value columns of a run on two workgroups while that gives every
-// workgroup a CU of its own.  64 chains, T = 4096, d = 128, a compaction every 64
-// tokens, one workgroup | two (with per-channel gates ahead) | the walk on 8:
-// bf16 2.55 | 2.44 | 2.71 ms, per-channel gates 2.79 | 2.57 | 2.79, float32 3.32 |
-// 2.95 | 3.19, with them 3.54 | 3.06 | 3.27.
-bool value_split(int D, int N, int nrun) { return D == 128 && (long long)N * nrun <= 128; }
-
 template <typename CT, int D, int P, int GL, int NVS>
-int launch_runs(const G3FwdArgs& a, int N, hipStream_t stream) {
+int launch_passes(const G3FwdArgs& a, int N, hipStream_t stream) {
   static_assert(sizeof(G3RunSmem<CT, D, P, GL, NVS>) <= 160 * 1024, "LDS budget");
   if (a.nrun > 1) {
     hipLaunchKernelGGL((gdn3_run_kernel<CT, D, P, GL, false, NVS>), dim3(N * (a.nrun - 1) * NVS), dim3(kNT), 0, stream, a);
@@ -597,16 +590,64 @@ int launch_runs(const G3FwdArgs& a, int N, hipStream_t stream) {
   return check_launch("gdn3_run_kernel");
 }
 
-template <typename CT, int D, int P>
-int launch_runs_gl(const G3FwdArgs& a, int N, hipStream_t stream) {
+// Runs of an interval of nsub sub-chunks: as many as the workgroups that run
+// at once (slots: two a CU, or one where LDS holds one) leave to a chain, each at
+// least a batch, and not so many that folding their maps takes longer than the two
+// scans of a run: a fold takes ~0.6 us a block of 16 slots squared, a batch 5
+// (bf16) to 9 us, so that sqrt(16 batches / blocks) is about the least sum.
+// Under four batches a single run: the second pass would cost what shorter
+// runs save.  T = 4096, d = 128, runs of at least two batches up to 512
+// workgroups | so | the walk on 8 workgroups: 64 chains, a compaction every 256
+// tokens, bf16 967 | 842 | 1112 us, float32 1351 | 1156 | 1629; 16 chains, float32,
+// every 320: 1300 | 762 | 1124; P = 64, 64 chains, bf16, every 1024 (one workgroup a
+// CU): 847 | 688 | 1141; two chains, T = 32768, none: 1471 | 396 | 6676.
+int interval_runs(int nsub, int N, int slots, int blocks) {
+  const int nb = (nsub + kBatch - 1) / kBatch;
+  if (nb < 4 || N >= slots) return 1;
+  int n = slots / N < nb ? slots / N : nb;
+  while (n > 1 && (long long)n * n * blocks > 16LL * nb) --n;
+  return n;
+}
+
+// One interval [c0, c1).  With several workgroups a chain the window state is
+// read from a.uw / a.vw by all of them and left in the other copy (a.uw_alt /
+// a.vw_alt), which then takes a.uw / a.vw's place; a single one updates it in
+// place.
+template <typename CT, int D, int P, int GL>
+int launch_runs(G3FwdArgs& a, int N, hipStream_t stream) {
+  constexpr int slots = sizeof(G3RunSmem<CT, D, P, GL, 1>) * 2 <= 160 * 1024 ? kG3RunTarget : kG3RunTarget / 2;
+  const int nsub = a.c1 - a.c0;
+  a.nrun = interval_runs(nsub, N, slots, P / kSC);
+  a.rlen = ((nsub + a.nrun - 1) / a.nrun + kBatch - 1) / kBatch * kBatch;
+  a.nrun = (nsub + a.rlen - 1) / a.rlen;
+  // The value columns of a run on two workgroups while each has a CU of its
+  // own.  64 chains, T = 4096, d = 128, a compaction every 64 tokens, one workgroup
+  // | two (with per-channel gates ahead) | the walk on 8: bf16 2.55 | 2.44 | 2.71
+  // ms, per-channel gates 2.79 | 2.57 | 2.79, float32 3.32 | 2.95 | 3.19, with them
+  // 3.54 | 3.06 | 3.27.
+  const bool split = D == 128 && N * a.nrun <= kG3RunTarget / 4;
+  const bool alt = a.nrun > 1 || split;
+  a.uw_out = alt ? a.uw_alt : a.uw;
+  a.vw_out = alt ? a.vw_alt : a.vw;
+  int rc;
   if constexpr (D == 128)
-    if (value_split(a.D, N, a.nrun))
-      return a.gate_ch > 1 ? launch_runs<CT, D, P, 2, 2>(a, N, stream) : launch_runs<CT, D, P, 1, 2>(a, N, stream);
-  return a.gate_ch > 1 ? launch_runs<CT, D, P, 2, 1>(a, N, stream) : launch_runs<CT, D, P, 1, 1>(a, N, stream);
+    rc = split ? launch_passes<CT, D, P, GL, 2>(a, N, stream) : launch_passes<CT, D, P, GL, 1>(a, N, stream);
+  else
+    rc = launch_passes<CT, D, P, GL, 1>(a, N, stream);
+  if (alt) {
+    std::swap(a.uw, a.uw_alt);
+    std::swap(a.vw, a.vw_alt);
+  }
+  return rc;
+}
+
+template <typename CT, int D, int P>
+int launch_runs_gl(G3FwdArgs& a, int N, hipStream_t stream) {
+  return a.gate_ch > 1 ? launch_runs<CT, D, P, 2>(a, N, stream) : launch_runs<CT, D, P, 1>(a, N, stream);
 }
 
 template <typename CT>
-int launch_runs_shape(const G3FwdArgs& a, int N, hipStream_t stream) {
+int launch_runs_shape(G3FwdArgs& a, int N, hipStream_t stream) {
   if (a.D == 128 && a.P == 16) return launch_runs_gl<CT, 128, 16>(a, N, stream);
   if (a.D == 128 && a.P == 32) return launch_runs_gl<CT, 128, 32>(a, N, stream);
   if (a.D == 128 && a.P == 64) return launch_runs_gl<CT, 128, 64>(a, N, stream);
@@ -616,12 +657,7 @@ int launch_runs_shape(const G3FwdArgs& a, int N, hipStream_t stream) {
   return set_error(GDNX_ERR_SHAPE, "gdn3: unsupported head_dim %d / P %d", a.D, a.P);
 }
 
-// Runs of an interval: enough workgroups over the chains to occupy the CUs
-// (kG3RunTarget), each run at least two batches (a run pays its first pass
-// and the fold of the runs before it).  At 64 chains over 2048-token intervals
-// 512 workgroups, two per CU as the registers allow: 1.96 ms the call; 256:
-// 2.32, 1024: 2.21.
-constexpr int kMinRun = 2 * kBatch;
+// the runs that any interval of N chains may be cut into
 int runs_max(int N) { return N >= kG3RunTarget ? 1 : kG3RunTarget / N; }
 
 }  // namespace
@@ -645,28 +681,8 @@ void gdn3_long_carve(G3FwdArgs& a, int N, char* w) {
   a.run_v = (float*)(w + 2 * win + g3_align256(n * a.P * a.D * 4));
 }
 
-// One interval [c0, c1).  With several workgroups a chain the window state is
-// read from a.uw / a.vw by all of them and left in the other copy (a.uw_alt /
-// a.vw_alt), which then takes a.uw / a.vw's place; a single one updates it in
-// place.
 int gdn3_long_interval(G3FwdArgs& a, int N, hipStream_t stream) {
-  const int nsub = a.c1 - a.c0;
-  int nrun = runs_max(N);
-  if (nrun > nsub / kMinRun) nrun = nsub / kMinRun;
-  if (nrun < 1) nrun = 1;
-  a.rlen = ((nsub + nrun - 1) / nrun + kBatch - 1) / kBatch * kBatch;
-  a.nrun = (nsub + a.rlen - 1) / a.rlen;
-  // (two workgroups of a chain read its window as one that may have ended has left it)
-  const bool alt = a.nrun > 1 || value_split(a.D, N, a.nrun);
-  a.uw_out = alt ? a.uw_alt : a.uw;
-  a.vw_out = alt ? a.vw_alt : a.vw;
-  const int rc = a.dtype == GDNX_DTYPE_BF16 ? launch_runs_shape<bf16>(a, N, stream)
-                                            : launch_runs_shape<float>(a, N, stream);
-  if (alt) {
-    std::swap(a.uw, a.uw_alt);
-    std::swap(a.vw, a.vw_alt);
-  }
-  return rc;
+  return a.dtype == GDNX_DTYPE_BF16 ? launch_runs_shape<bf16>(a, N, stream) : launch_runs_shape<float>(a, N, stream);
 }
 
 }  // namespace gdnx

@@ -321,7 +321,7 @@ int gdn3_fwd_dispatch(const G3FwdArgs& a, hipStream_t stream);
 bool gdn3_fwd_fused(int D, int P, int Kc, int dtype);
 // bytes of the static scratch of gdnx_gdn3_chunk_fwd_state_noalloc (per device)
 constexpr size_t kG3ScratchBytes = (size_t)64 << 20;
-// workgroups an interval is spread over (chains x runs)
+// workgroups an interval is spread over (chains x runs) at most: two a CU
 constexpr int kG3RunTarget = 512;
 // that scratch's address on the current device (resolved once per device)
 int gdn3_scratch(void** out);

@@ -317,7 +317,8 @@ __device__ __forceinline__ float pick4(const f32x4& x, int i) {
 
 // SCORE (|r_t| requested): each value tile's sum of squares of a token's net
 // write goes to the record's U, at the tile's first column, which only this
-// workgroup reads and has read; chan_rnorm_kernel sums them.
+// workgroup reads and has read; chan_rnorm_kernel sums them.  A workgroup that
+// has all value columns (d = 64, four tiles) writes |r_t| itself.
 template <int D, int NV, bool STASH, bool SCORE>
 __global__ void __launch_bounds__(256, 2) chan_split_fwd_kernel(ChanArgs p) {
   typedef ChRec<D> Rc;
@@ -421,7 +422,7 @@ __global__ void __launch_bounds__(256, 2) chan_split_fwd_kernel(ChanArgs p) {
           float* rst = (float*)p.chunk_states + NR * D * D + rec * (CC * D);
           *(f32x4*)(rst + stash_tile_offset<float, D>(0, V0 + v, lane)) = R[v];
         }
-      if constexpr (SCORE)
+      if constexpr (SCORE && NV < Sp::NVT)
         if (wave == 0) {   // (U's reader)
           float* fr = p.frec + rec * Rc::FN;
           const f32x4 sq = R[v] * R[v];
@@ -432,6 +433,18 @@ __global__ void __launch_bounds__(256, 2) chan_split_fwd_kernel(ChanArgs p) {
           }
         }
     }
+    if constexpr (SCORE && NV == Sp::NVT)
+      if (wave == (c & 3)) {   // all value columns are here
+        f32x4 sq = zero4();
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sq += R[v] * R[v];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float n2 = row_prefix16(sq[e]);
+          const int t = c * CC + 4 * g4 + e;
+          if (n16 == 15 && t < p.T) p.r_norm[((size_t)b * p.T + t) * p.H + h] = sqrtf(n2);
+        }
+      }
   };
   Ops x[PF];
 #pragma unroll
@@ -848,6 +861,11 @@ static int chan_tiles(int nchains, int D) {
   return tiles <= 256 ? 1 : tiles < 1024 ? 2 : 4;
 }
 
+// Up to this many chunks four tiles a workgroup, which need no launch for |r_t|
+// after the scan, are at d = 64 no slower than the narrower split (2 chains, T =
+// 16: 86 -> 82 us a scored call; at 128 tokens 84 -> 88, so no more).
+constexpr int kScoreChunks = 4;
+
 template <int D, int NV>
 static int launch_chan_scan(const ChanArgs& a, hipStream_t stream) {
   const dim3 grid(a.B * a.H * (ChSplit<D>::NVT / NV)), block(256);
@@ -873,10 +891,11 @@ static int launch_chan_fwd(ChanArgs a, hipStream_t stream) {
     hipLaunchKernelGGL((chan_prep_kernel<D, false>), dim3(nchains * NC), dim3(64 * (D / 16)), 0, stream, a);
   int rc = check_launch("chan_prep_kernel");
   if (rc) return rc;
-  const int nv = chan_tiles(nchains, D);
+  int nv = chan_tiles(nchains, D);
+  if (a.r_norm && D == 64 && NC <= kScoreChunks) nv = 4;
   rc = nv == 1 ? launch_chan_scan<D, 1>(a, stream)
                : nv == 2 ? launch_chan_scan<D, 2>(a, stream) : launch_chan_scan<D, 4>(a, stream);
-  if (rc || !a.r_norm) return rc;
+  if (rc || !a.r_norm || nv == ChSplit<D>::NVT) return rc;
   const long long n = (long long)nchains * a.T;
   hipLaunchKernelGGL((chan_rnorm_kernel<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a);
   return check_launch("chan_rnorm_kernel");

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 # a workgroup change on 256 CUs (d = 128: 33 and 128, d = 64: 65 and 256)
 CASES = [(1, 1, 128, 1), (1, 2, 128, 16), (2, 1, 64, 17), (1, 2, 64, 64), (1, 1, 128, 65), (1, 2, 128, 130),
          (2, 16, 128, 33), (3, 11, 128, 63), (3, 11, 128, 97), (8, 16, 128, 31), (8, 16, 128, 50), (5, 13, 64, 65),
-         (16, 16, 64, 49), (16, 16, 64, 1)]
+         (16, 16, 64, 49), (16, 16, 64, 1), (16, 16, 64, 90)]
 
 
 @pytest.mark.parametrize("B,H,D,T", CASES)

@@ -769,10 +769,8 @@ template <typename CT> struct G3Raw {
 };
 
 // local token t (marked invalid outside [0, T) or for a thread without a
-// unit; the loads then read token min(max(t, 0), T - 1)).  GL: the gate
-// layout, 1 a scalar per lane, 2 per channel, 0 read from o.gc (a runtime
-// branch, whose merge costs the prefetch a wait)
-template <typename CT, int GL = 0>
+// unit; the loads then read token min(max(t, 0), T - 1))
+template <typename CT>
 __device__ __forceinline__ void g3_fetch(const G3FwdArgs& p, const G3Tok& o, G3Raw<CT>& r, int t, bool on,
                                          int ud) {
   constexpr int W16 = W16Of<CT>::value;
@@ -788,18 +786,18 @@ __device__ __forceinline__ void g3_fetch(const G3FwdArgs& p, const G3Tok& o, G3R
     r.v[w] = vp[w];
   }
   // both branches define every gate field, so no loaded register is merged
-  if (GL == 2 || (GL == 0 && o.gc > 1)) {
+  if (o.gc > 1) {
     const float* bp = p.bg + o.gate_base + tc * o.gate_tok + ud;
     const float* wp = p.wg + o.gate_base + tc * o.gate_tok + ud;
     r.b0 = *(const f32x4*)bp;
     r.b1 = *(const f32x4*)(bp + 4);
     r.w0 = *(const f32x4*)wp;
     r.w1 = *(const f32x4*)(wp + 4);
-    if constexpr (GL == 0) r.bs = r.ws = 0.f;
+    r.bs = r.ws = 0.f;
   } else {
     r.bs = p.bg[o.gate_base + tc * o.gate_tok];
     r.ws = p.wg[o.gate_base + tc * o.gate_tok];
-    if constexpr (GL == 0) r.b0 = r.b1 = r.w0 = r.w1 = zero4();
+    r.b0 = r.b1 = r.w0 = r.w1 = zero4();
   }
   r.dec = p.dec[o.dec_base + tc * o.dec_tok];
 }
@@ -812,12 +810,12 @@ __device__ __forceinline__ uint4 g3_raw(const G3Raw<CT>& r, const uint4& x) {
 
 // h = b o k and u = w o v of the thread's 8 channels (gc: gate channels);
 // returns the row sum of k . h over the token's DG threads (consecutive lanes)
-template <typename CT, int DG, int GL = 0>
+template <typename CT, int DG>
 __device__ __forceinline__ float g3_unpack(const G3Raw<CT>& r, int gc, float* hf, float* uu) {
   float kf[8], vf[8], bb[8], ww[8];
   unpack8(r.k, kf, (const CT*)nullptr);
   unpack8(r.v, vf, (const CT*)nullptr);
-  if (GL == 2 || (GL == 0 && gc > 1)) {
+  if (gc > 1) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       bb[e] = r.b0[e];
@@ -859,23 +857,22 @@ __device__ __forceinline__ float g3_unpack(const G3Raw<CT>& r, int gc, float* hf
 
 // The window LDS a sub-chunk step works on (pointers into one workgroup's
 // shared memory)
-template <typename CT, int D, int P>
+template <typename CT, int D>
 struct G3WinView {
   CT (*x)[D + 8];               // rows: H (0..15), Q (16..31), K (32..47)
   float (*u)[D + 4];            // w (.) v
   float (*kr)[D + 4];           // Kronecker reads of H and Q
   float (*pp)[kSC][kSC + 4];    // [4]: H K^T (then inverse scratch), Aq, T, inverse scratch
-  float (*po)[kSC][P + 4];      // [2]: Ho, Qo over the P slots
+  float (*po)[kSC][kSC + 4];    // [2]: Ho, Qo over the slots
   CT (*skron)[D + 8];           // this workgroup's rows of sum_r A_r (x) B_r
-  float (*vbd)[D + 4];          // window keys: block b decayed to e^{-boff_b} of now
+  float (*vbd)[D + 4];          // window keys, decayed to now
   CT (*vbx)[D + 8];             // the same in the compute dtype (bf16 IO)
   float *G, *alpha, *lg, *kco, *qco, *gam, *vsc;
-  float* boff;                  // log decay of block b's keys since they were rebased
 };
 
 // The log-decay prefix sums of a sub-chunk (lane i < 16 holds G_i).
-template <typename CT, int D, int P>
-__device__ __forceinline__ float g3_scan_g(const G3WinView<CT, D, P>& w, int lane) {
+template <typename CT, int D>
+__device__ __forceinline__ float g3_scan_g(const G3WinView<CT, D>& w, int lane) {
   float gl = lane < kSC ? w.lg[lane] : 0.f;
 #pragma unroll
   for (int off = 1; off < kSC; off <<= 1) {
@@ -887,8 +884,8 @@ __device__ __forceinline__ float g3_scan_g(const G3WinView<CT, D, P>& w, int lan
 
 // The per-token coefficients of a sub-chunk (one wave): G, e^G, kco = alpha
 // e^{2 (gacc + G)}, qco = e^{2 (gacc + G)} and the key scale e^{G_last - G}.
-template <typename CT, int D, int P>
-__device__ __forceinline__ void g3_scalars(const G3WinView<CT, D, P>& w, float gl, float gacc, int lane) {
+template <typename CT, int D>
+__device__ __forceinline__ void g3_scalars(const G3WinView<CT, D>& w, float gl, float gacc, int lane) {
   const float gl_last = __shfl(gl, kSC - 1, 64);
   if (lane < kSC) {
     const float e2 = expf(2.f * (gacc + gl));
@@ -900,13 +897,12 @@ __device__ __forceinline__ void g3_scalars(const G3WinView<CT, D, P>& w, float g
   }
 }
 
-// Gram tile ti of a sub-chunk (one wave; 2 + 2 NB tiles):
+// Gram tile ti of a sub-chunk (one wave; 4 tiles):
 //   0: H K^T (raw; the inverse turns it into T),  1: Aq = [j <= i] e^{G_i - G_j} q_i.k_j,
-//   2 + 2 b: Ho_b = vis alpha_i e^{G_i + boff_b} h_i.Vb_b[j],  3 + 2 b: Qo_b = vis e^{G_i + boff_b} q_i.Vb_b[j]
-// with vis = [b != beta or j >= i or j < lo]
-template <typename CT, int D, int P>
-__device__ __forceinline__ void g3_gram_tile(const G3WinView<CT, D, P>& w, int ti, float gl, int beta, int lo,
-                                             int lane) {
+//   2: Ho = vis alpha_i e^{G_i} h_i.Vb[j],        3: Qo = vis e^{G_i} q_i.Vb[j]
+// with vis = [j >= i or j < lo]
+template <typename CT, int D>
+__device__ __forceinline__ void g3_gram_tile(const G3WinView<CT, D>& w, int ti, float gl, int lo, int lane) {
   constexpr bool KF = sizeof(CT) == 4;
   const int g4 = lane >> 4, n16 = lane & 15;
   const float gj = __shfl(gl, n16, 64);
@@ -915,11 +911,10 @@ __device__ __forceinline__ void g3_gram_tile(const G3WinView<CT, D, P>& w, int t
   for (int s = 0; s < 4; ++s) gi[s] = __shfl(gl, 4 * g4 + s, 64);
   const bool isq = ti & 1;
   const CT* arow = &w.x[(isq ? kSC : 0) + n16][0];
-  const int bl = (ti - 2) >> 1;
   const CT* brow;
   if (ti < 2) brow = &w.x[2 * kSC + n16][0];
-  else if constexpr (KF) brow = (const CT*)&w.vbd[kSC * bl + n16][0];
-  else brow = &w.vbx[kSC * bl + n16][0];
+  else if constexpr (KF) brow = (const CT*)&w.vbd[n16][0];
+  else brow = &w.vbx[n16][0];
   const f32x4 acc = tile_nt<CT, D>(arow, brow, g4);
   const int j = n16;
   if (ti == 0) {
@@ -932,13 +927,12 @@ __device__ __forceinline__ void g3_gram_tile(const G3WinView<CT, D, P>& w, int t
       w.pp[1][i][j] = (j <= i) ? expf(gi[s] - gj) * acc[s] : 0.f;
     }
   } else {
-    const float bo = w.boff[bl];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int i = 4 * g4 + s;
-      const bool vis = bl != beta || j >= i || j < lo;
-      const float sc = expf(gi[s] + bo) * (isq ? 1.f : w.alpha[i]);
-      w.po[isq ? 1 : 0][i][kSC * bl + j] = vis ? sc * acc[s] : 0.f;
+      const bool vis = j >= i || j < lo;
+      const float sc = expf(gi[s]) * (isq ? 1.f : w.alpha[i]);
+      w.po[isq ? 1 : 0][i][j] = vis ? sc * acc[s] : 0.f;
     }
   }
 }
@@ -949,8 +943,8 @@ __device__ __forceinline__ void g3_gram_tile(const G3WinView<CT, D, P>& w, int t
 // (nilpotent): (I + Lm)^-1 = (I - L)(I + L^2)(I + L^4)(I + L^8), factors that
 // commute; squarings and products on fp32 MFMA.  An accumulator tile is a
 // k-fragment (B operand); the A operand of each square goes through LDS.
-template <typename CT, int D, int P>
-__device__ __forceinline__ void g3_inverse(const G3WinView<CT, D, P>& w, int lane) {
+template <typename CT, int D>
+__device__ __forceinline__ void g3_inverse(const G3WinView<CT, D>& w, int lane) {
   const int g4 = lane >> 4, n16 = lane & 15;
   wave_lds_sync();
   f32x4 xa, ta;
@@ -982,8 +976,8 @@ __device__ __forceinline__ void g3_inverse(const G3WinView<CT, D, P>& w, int lan
 // The commit of a sub-chunk's prefetched token rows into the window LDS: H =
 // b (.) k, the Q and K rows, u = w (.) v, and per token alpha and the log
 // decay (thread tid holds load unit (tid / (D / 8), 8 (tid mod (D / 8)))).
-template <typename CT, int D, int P>
-__device__ __forceinline__ void g3_commit(const G3WinView<CT, D, P>& w, const G3Tok& tk, const G3Raw<CT>& r, int tid) {
+template <typename CT, int D>
+__device__ __forceinline__ void g3_commit(const G3WinView<CT, D>& w, const G3Tok& tk, const G3Raw<CT>& r, int tid) {
   constexpr int DG = D / 8, W16 = W16Of<CT>::value;
   if (tid >= kSC * DG) return;
   const int ui = tid / DG, ud = 8 * (tid % DG);
@@ -1011,11 +1005,11 @@ __device__ __forceinline__ void g3_commit(const G3WinView<CT, D, P>& w, const G3
 // the coefficients, H K^T and the inverse, wave 2 Aq and wave 3 the window
 // grams.  The commit's x, u and scalars and the tiles' pp, po must lie in LDS
 // the compaction no longer uses.
-template <typename CT, int D, int P>
-__device__ __forceinline__ void g3_stage_a_shadow(const G3WinView<CT, D, P>& w, const G3FwdArgs& p,
+template <typename CT, int D>
+__device__ __forceinline__ void g3_stage_a_shadow(const G3WinView<CT, D>& w, const G3FwdArgs& p,
                                                   const G3Tok& tk, G3Raw<CT>& ra, G3Raw<CT>& rb, int c,
                                                   int wave, int lane) {
-  constexpr int NB = P / kSC, DG = D / 8, PASSES = kSC * DG / 64;
+  constexpr int DG = D / 8, PASSES = kSC * DG / 64;
   static_assert(PASSES % 2 == 0, "load passes in pairs");
   auto fetch = [&](G3Raw<CT>& r, int pass) {
     const int u = pass * 64 + lane;
@@ -1025,83 +1019,64 @@ __device__ __forceinline__ void g3_stage_a_shadow(const G3WinView<CT, D, P>& w, 
   for (int pass = 0; pass < PASSES; pass += 2) {
     fetch(ra, pass);
     fetch(rb, pass + 1);
-    g3_commit<CT, D, P>(w, tk, ra, pass * 64 + lane);
-    g3_commit<CT, D, P>(w, tk, rb, (pass + 1) * 64 + lane);
+    g3_commit<CT, D>(w, tk, ra, pass * 64 + lane);
+    g3_commit<CT, D>(w, tk, rb, (pass + 1) * 64 + lane);
   }
   wave_lds_sync();
-  const int lo = max(0, p.t0 - c * kSC), beta = c % NB;
+  const int lo = max(0, p.t0 - c * kSC);
   const float gl = g3_scan_g(w, lane);
   if (wave == 1) {
     g3_scalars(w, gl, 0.f, lane);
-    g3_gram_tile<CT, D, P>(w, 0, gl, beta, lo, lane);
+    g3_gram_tile<CT, D>(w, 0, gl, lo, lane);
     g3_inverse(w, lane);
   } else if (wave == 2) {
-    g3_gram_tile<CT, D, P>(w, 1, gl, beta, lo, lane);
+    g3_gram_tile<CT, D>(w, 1, gl, lo, lane);
   } else {
 #pragma unroll
-    for (int ti = 2; ti < 2 + 2 * NB; ++ti) g3_gram_tile<CT, D, P>(w, ti, gl, beta, lo, lane);
+    for (int ti = 2; ti < 4; ++ti) g3_gram_tile<CT, D>(w, ti, gl, lo, lane);
   }
 }
 
-// One sub-chunk c of the single-stage window recurrence for one workgroup
-// (value tiles vb NVTW .. of chain): commit of its prefetched token rows (and
-// the loads of sub-chunk next, if >= 0), the grams, the inverse, the
-// Kronecker reads, the window algebra on the U tiles uo, y and the training
-// stash, then the window keys.  first: no sub-chunk before it in this launch;
-// committed: its token rows are in LDS already (g3_commit ran earlier).
-template <typename CT, int D, int P, int NVB>
-__device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, const G3FwdArgs& p, const G3Tok& tk,
-                                               int chain, int vb, int c, bool first, int next, bool live,
-                                               float& gacc, f32x4 (&uo)[P / kSC][(D / 16 / NVB + 3) / 4],
-                                               G3Raw<CT>& raw, bool committed = false) {
-  constexpr int NB = P / kSC;
+// Sub-chunk c of the window recurrence, a chain a workgroup: commit of its
+// prefetched token rows, the grams, the inverse, the Kronecker reads, the
+// window algebra on the U tiles uo, y and the training stash, then the window
+// keys.  committed: its token rows are in LDS already (g3_commit ran earlier).
+template <typename CT, int D>
+__device__ __forceinline__ void g3_window_step(const G3WinView<CT, D>& w, const G3FwdArgs& p, const G3Tok& tk,
+                                               int chain, int c, bool live, float& gacc,
+                                               f32x4 (&uo)[(D / 16 + 3) / 4], const G3Raw<CT>& raw, bool committed) {
   constexpr bool KF = sizeof(CT) == 4;
   constexpr int DG = D / 8;  // 8-element load units per token row
-  constexpr int UNITS = kSC * DG;
   constexpr int W16 = W16Of<CT>::value;
   constexpr int KS = FragT<CT>::KSTEP;
   typedef typename FragT<CT>::type Frag;
-  constexpr int NVTW = D / 16 / NVB;   // value tiles of this workgroup: vb NVTW + [0, NVTW)
-  constexpr int VPW = (NVTW + 3) / 4;
+  constexpr int NVT = D / 16, VPW = (NVT + 3) / 4;   // value tiles, per wave
   const int tid = opaque(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g4 = lane >> 4, n16 = lane & 15;
   const int T = p.T;
-  const bool has_unit = tid < UNITS;
-  const int ui = tid / DG, ud = 8 * (tid % DG);
-  auto fetch = [&](G3Raw<CT>& r, int cc) { g3_fetch<CT>(p, tk, r, cc * kSC + ui - p.t0, has_unit, ud); };
-  auto commit = [&](const G3Raw<CT>& r) { g3_commit<CT, D, P>(w, tk, r, tid); };
-  // after sub-chunk cc: its block is rebased (boff 0), the others decayed by its G_last
-  auto advance_boff = [&](int cc, float glast) {
-    if (tid < NB) w.boff[tid] = (tid == cc % NB) ? 0.f : w.boff[tid] + glast;
-  };
-  auto vown = [&](int a) { return wave + 4 * a < NVTW; };
-  auto vtile = [&](int a) { return vb * NVTW + wave + 4 * a; };
+  auto vown = [&](int a) { return wave + 4 * a < NVT; };
+  auto vtile = [&](int a) { return wave + 4 * a; };
 
-    // slots [lo, hi) of block beta receive this call's tokens; the others (the
+    // slots [lo, hi) receive this call's tokens; the others (the
     // head a previous call wrote, the tail after the last token) keep the
     // writes they hold and stay visible to every token of the sub-chunk
     const int lo = max(0, p.t0 - c * kSC), hi = min(kSC, p.t0 + T - c * kSC);
-    const int beta = c % NB;
     __syncthreads();
-    if (!first) advance_boff(c - 1, w.G[kSC - 1]);
-    if (!committed) commit(raw);
-    if (next >= 0) fetch(raw, next);
+    if (!committed) g3_commit<CT, D>(w, tk, raw, tid);
     __syncthreads();
     // per-token scalars | grams and Kronecker reads (MFMA).  Every wave forms
     // the log-decay prefix sums G (lane i holds G_i); wave 0 publishes the
-    // per-token coefficients, the gram tiles go round the waves, and wave 0
+    // per-token coefficients, each wave forms a gram tile, and wave 0
     // forms the inverse while waves 1..3 do the Kronecker reads.  A committed
     // sub-chunk had all of this formed in the previous compaction's shadow.
     if (!committed) {
       const float gl = g3_scan_g(w, lane);
       if (wave == 0) g3_scalars(w, gl, gacc, lane);
-#pragma unroll
-      for (int r = 0; r < (2 + 2 * NB + 3) / 4; ++r)
-        if (wave + 4 * r < 2 + 2 * NB) g3_gram_tile<CT, D, P>(w, wave + 4 * r, gl, beta, lo, lane);
+      g3_gram_tile<CT, D>(w, wave, gl, lo, lane);
       if (wave == 0) g3_inverse(w, lane);
     }
     if (live && (committed || wave > 0)) {
-      // this workgroup's value tiles over waves 1..3 (wave 0 forms the inverse), or all four
+      // the value tiles over waves 1..3 (wave 0 forms the inverse), or all four
       const int w0 = committed ? wave : wave - 1, ws = committed ? 4 : 3;
       // the H and Q fragments serve every value tile; each tile's Kronecker
       // fragments are read ahead of its MFMAs behind a scheduling barrier (the
@@ -1111,11 +1086,10 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
       for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
         for (int kb = 0; kb < D / KS; ++kb) xf[rt][kb] = ld_frag(&w.x[rt * 16 + n16][kb * KS], g4);
-      for (int l = w0; l < NVTW; l += ws) {
-        const int vt = vb * NVTW + l;
+      for (int vt = w0; vt < NVT; vt += ws) {
         Frag bf[D / KS];
 #pragma unroll
-        for (int kb = 0; kb < D / KS; ++kb) bf[kb] = ld_frag(&w.skron[l * 16 + n16][kb * KS], g4);
+        for (int kb = 0; kb < D / KS; ++kb) bf[kb] = ld_frag(&w.skron[vt * 16 + n16][kb * KS], g4);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
@@ -1129,17 +1103,12 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
     }
     __syncthreads();
     // window algebra on fp32 MFMA, per wave its VPW value tiles:
-    //   Rhs = alpha u - kco KRh - sum_b Ho_b U_b;  U = T Rhs
-    //   Y   = qco KRq + sum_b Qo_b U_b + Aq U
+    //   Rhs = alpha u - kco KRh - Ho U_old;  U = T Rhs
+    //   Y   = qco KRq + Qo U_old + Aq U
     // (an accumulator tile over rows = tokens is directly a k-fragment)
     // (every LDS operand read ahead, behind a scheduling barrier; the
     // coefficient tiles and per-token scalars serve every value tile)
-    f32x4 po0[NB], po1[NB];
-#pragma unroll
-    for (int bl = 0; bl < NB; ++bl) {
-      po0[bl] = *(const f32x4*)&w.po[0][n16][kSC * bl + 4 * g4];
-      po1[bl] = *(const f32x4*)&w.po[1][n16][kSC * bl + 4 * g4];
-    }
+    const f32x4 po0 = *(const f32x4*)&w.po[0][n16][4 * g4], po1 = *(const f32x4*)&w.po[1][n16][4 * g4];
     const f32x4 ptf = *(const f32x4*)&w.pp[2][n16][4 * g4], paf = *(const f32x4*)&w.pp[1][n16][4 * g4];
     float alv[4], kcv[4], qcv[4], uv[VPW][4], khv[VPW][4], kqv[VPW][4];
 #pragma unroll
@@ -1167,8 +1136,7 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
       if (!vown(a)) continue;
       const int v = vtile(a) * 16 + n16;
       f32x4 acc = zero4();
-#pragma unroll
-      for (int bl = 0; bl < NB; ++bl) mma(acc, po0[bl], uo[bl][a]);
+      mma(acc, po0, uo[a]);
       f32x4 rhs;
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
@@ -1179,8 +1147,7 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
       f32x4 un = zero4();
       mma(un, ptf, rhs);
       f32x4 yv = zero4();
-#pragma unroll
-      for (int bl = 0; bl < NB; ++bl) mma(yv, po1[bl], uo[bl][a]);
+      mma(yv, po1, uo[a]);
       mma(yv, paf, un);
       CT* yp = (CT*)p.y + tk.y_base + v;
 #pragma unroll
@@ -1192,27 +1159,24 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
         if (t >= 0 && t < T) yp[(size_t)t * tk.y_tok] = from_f<CT>(out);
       }
 #pragma unroll
-      for (int bl = 0; bl < NB; ++bl)
-        if (bl == beta)
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            const int i = 4 * g4 + s;
-            if (i >= lo && i < hi) uo[bl][a][s] = un[s];
-          }
+      for (int s = 0; s < 4; ++s) {
+        const int i = 4 * g4 + s;
+        if (i >= lo && i < hi) uo[a][s] = un[s];
+      }
       if (p.ts_u) {   // training stash: this sub-chunk's net writes
         float* us = p.ts_u + ((size_t)chain * p.nch + c) * kSC * D + v;
 #pragma unroll
         for (int s = 0; s < 4; ++s) us[(size_t)(4 * g4 + s) * D] = un[s];
       }
     }
-    if (p.ts_g && tid == 0 && vb == 0) p.ts_g[(size_t)chain * p.nch + c] = gacc;
-    // block beta's keys for the next sub-chunks: the slots this sub-chunk
-    // wrote take k_j decayed to its end, the others their old keys decayed
-    // over it (8 consecutive keys per thread); the block's offset restarts
+    if (p.ts_g && tid == 0) p.ts_g[(size_t)chain * p.nch + c] = gacc;
+    // the keys for the next sub-chunk: the slots this one wrote take k_j decayed
+    // to its end, the others their old keys decayed over it (8 consecutive keys
+    // per thread)
     {
-      const float olds = expf(w.boff[beta] + w.G[kSC - 1]);
+      const float olds = expf(w.G[kSC - 1]);
       for (int u8 = tid; u8 < kSC * D / 8; u8 += kNT) {
-        const int j = u8 / DG, d = 8 * (u8 % DG), sl = kSC * beta + j;
+        const int j = u8 / DG, d = 8 * (u8 % DG);
         uint4 kw[W16];
 #pragma unroll
         for (int q16 = 0; q16 < W16; ++q16) kw[q16] = *(const uint4*)&w.x[2 * kSC + j][d + q16 * (16 / sizeof(CT))];
@@ -1221,15 +1185,15 @@ __device__ __forceinline__ void g3_window_step(const G3WinView<CT, D, P>& w, con
         float sc = w.vsc[j];
         if (j < lo || j >= hi) {
           sc = olds;
-          const f32x4 o0 = *(const f32x4*)&w.vbd[sl][d], o1 = *(const f32x4*)&w.vbd[sl][d + 4];
+          const f32x4 o0 = *(const f32x4*)&w.vbd[j][d], o1 = *(const f32x4*)&w.vbd[j][d + 4];
           kf[0] = o0[0], kf[1] = o0[1], kf[2] = o0[2], kf[3] = o0[3];
           kf[4] = o1[0], kf[5] = o1[1], kf[6] = o1[2], kf[7] = o1[3];
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) kf[e] *= sc;
-        *(f32x4*)&w.vbd[sl][d] = (f32x4){kf[0], kf[1], kf[2], kf[3]};
-        *(f32x4*)&w.vbd[sl][d + 4] = (f32x4){kf[4], kf[5], kf[6], kf[7]};
-        if constexpr (!KF) store8(&w.vbx[sl][d], kf);
+        *(f32x4*)&w.vbd[j][d] = (f32x4){kf[0], kf[1], kf[2], kf[3]};
+        *(f32x4*)&w.vbd[j][d + 4] = (f32x4){kf[4], kf[5], kf[6], kf[7]};
+        if constexpr (!KF) store8(&w.vbx[j][d], kf);
       }
     }
     gacc += w.G[kSC - 1];
@@ -1308,7 +1272,6 @@ struct G3FusedSmem {
   alignas(16) float uwin[P][D + 4];     // the window's net writes (slot-major)
   alignas(16) float vbd[P][D + 4];      // its keys, decayed to now
   alignas(16) CT vbx[sizeof(CT) == 4 ? 1 : P][D + 8];
-  float boff[1];
 };
 template <typename CT, int D>
 constexpr bool fused_fits() { return sizeof(G3FusedSmem<CT, D>) <= 160 * 1024; }
@@ -1346,7 +1309,6 @@ __global__ void __launch_bounds__(kNT) gdn3_fused_kernel(G3FwdArgs p) {
     sm.vbd[j][d] = kv;
     if constexpr (sizeof(CT) == 2) sm.vbx[j][d] = from_f<CT>(kv);
   }
-  if (tid == 0) sm.boff[0] = 0.f;
   __syncthreads();
   if (carried) write_skron<D, CT>(&sm.ph.w.skron[0][0], sm.ab, sm.ab + Rm, tid, D + 8);
   bool live = carried;
@@ -1356,10 +1318,10 @@ __global__ void __launch_bounds__(kNT) gdn3_fused_kernel(G3FwdArgs p) {
   G3Raw<CT> raw2;
   float gacc = 0.f;
   int event = 0;
-  const G3WinView<CT, D, P> w{sm.ph.w.x, sm.ph.w.u, sm.ph.w.kr, sm.ph.w.pp, sm.ph.w.po, sm.ph.w.skron, sm.vbd,
-                              sm.vbx, sm.ph.w.G, sm.ph.w.alpha, sm.ph.w.lg, sm.ph.w.kco, sm.ph.w.qco,
-                              sm.ph.w.gam, sm.ph.w.vsc, sm.boff};
-  f32x4 uo[1][VPW];
+  const G3WinView<CT, D> w{sm.ph.w.x, sm.ph.w.u, sm.ph.w.kr, sm.ph.w.pp, sm.ph.w.po, sm.ph.w.skron, sm.vbd,
+                           sm.vbx, sm.ph.w.G, sm.ph.w.alpha, sm.ph.w.lg, sm.ph.w.kco, sm.ph.w.qco,
+                           sm.ph.w.gam, sm.ph.w.vsc};
+  f32x4 uo[VPW];
   // the chain's sketch, the same at every compaction, held from here (a load
   // per compaction waited, in order, for the window's output stores before it)
   G3Sketch<D> sk;
@@ -1375,15 +1337,15 @@ __global__ void __launch_bounds__(kNT) gdn3_fused_kernel(G3FwdArgs p) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int vt = wave + 4 * a;
-        uo[0][a][s] = vt < D / 16 ? sm.uwin[4 * g4 + s][vt * 16 + n16] : 0.f;
+        uo[a][s] = vt < D / 16 ? sm.uwin[4 * g4 + s][vt * 16 + n16] : 0.f;
       }
-    g3_window_step<CT, D, P, 1>(w, p, tk, chain, 0, c, true, -1, live, gacc, uo, raw, committed);
+    g3_window_step<CT, D>(w, p, tk, chain, c, live, gacc, uo, raw, committed);
 #pragma unroll
     for (int a = 0; a < VPW; ++a)
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int vt = wave + 4 * a;
-        if (vt < D / 16) sm.uwin[4 * g4 + s][vt * 16 + n16] = uo[0][a][s];
+        if (vt < D / 16) sm.uwin[4 * g4 + s][vt * 16 + n16] = uo[a][s];
       }
     const bool complete = (long long)(c + 1) * kSC <= tend;
     __syncthreads();
@@ -1397,7 +1359,7 @@ __global__ void __launch_bounds__(kNT) gdn3_fused_kernel(G3FwdArgs p) {
     // is added to the eigen-solve's wave)
     auto issue = [&]() {};
     auto commit = [&]() {
-      if (pre && wave > 0) g3_stage_a_shadow<CT, D, P>(w, p, tk, raw, raw2, c + 1, wave, lane);
+      if (pre && wave > 0) g3_stage_a_shadow<CT, D>(w, p, tk, raw, raw2, c + 1, wave, lane);
     };
     g3_compact<D, P>(sm.ph.cs, sm.ab, &sm.uwin[0][0], &sm.vbd[0][0], (size_t)(D + 4), (size_t)1, gacc, p.sdec,
                      p.sketch + (size_t)chain * Ge::n * qs,

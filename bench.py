@@ -493,7 +493,8 @@ def bench_gdn3(args, layer_default, train=False):
         "roofline": {"bound": "hbm", "kernel": name, "achieved": achieved, "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": achieved * 1e9 / HBM_PEAK, "traffic": measured_traffic(name),
                      "mean_us": sec * 1e6, "algorithmic_bytes": nbytes,
-                     "note": "one workgroup per chain walks the windows in order: latency-bound"},
+                     "note": "one workgroup per chain walks the windows in order: latency-bound" if layer_default else
+                             "the intervals in order, each two passes over its runs and a compaction: latency-bound"},
         "finite": bool(torch.isfinite(y.float()).all()),
     }
     if not args.no_cpu_baseline:

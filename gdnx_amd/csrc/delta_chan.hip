@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(64 * (D / 16), D == 128 ? 4 : 3) chan_prep_ker
 // into MFMA fragments, PF chunks ahead, and a step has one barrier.  With few
 // chains a step is bound by its latency: the fp32 MFMAs (16 x 16 x 4, 32
 // cycles) over D / 4 keys, then the exchange.  d = 128: B = 2, T = 512, H = 16
-// with stash, forward / reverse 105 / 90 us with only the value columns split,
+// with stash, forward / reverse 103 / 90 us with only the value columns split,
 // 43 / 45 us so (49 / 51 us while a step could wait for a later chunk's
 // loads); B = 1, T = 2048 forward 292 us, then 125 us.
 // ---------------------------------------------------------------------------
@@ -851,11 +851,11 @@ __global__ void __launch_bounds__(64 * (D / 16), D == 128 ? 4 : 3) chan_grads_ke
 // Value tiles per workgroup of the scans: one while each of the 256 CUs
 // gets one workgroup at most (the step's latency counts), two up to two full
 // rounds of the chip, four beyond (a record is read D / 64 times instead of D / 16, and
-// more products stand between two barriers).  Times of the
-// whole call, the gradient kernel at 108 us per 32 chains then, T = 512 training
-// (1 | 2 | 4 tiles) at d = 128:
-// 64 chains 512 | 488 | 548 us, 96: 750 | 728 | 717, 128: 971 | 887 | 864, 256:
-// 1829 | 1670 | 1574; T = 1024 without gradient, 64 chains 328 | 320 | 389.
+// more products stand between two barriers).  The whole call, T = 512, training
+// (1 | 2 | 4 tiles) at d = 128: 32 chains 231 | 262 | 331 us, 48: 344 | 322 | 389,
+// 64: 423 | 398 | 458, 96: 612 | 586 | 571, 128: 781 | 693 | 673, 256: 1509 | 1337 |
+// 1244; at d = 64, 64 chains 182 | 210 | 256, 128: 341 | 321 | 360, 256: 632 | 577 |
+// 550.
 static int chan_tiles(int nchains, int D) {
   const long long tiles = (long long)nchains * (D / 16);
   return tiles <= 256 ? 1 : tiles < 1024 ? 2 : 4;
